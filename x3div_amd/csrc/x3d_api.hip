@@ -222,6 +222,25 @@ static int upload_tables(x3d_ctx* c)
   return X3D_OK;
 }
 
+int fused_plans(x3d_ctx* c, long long pts)
+{
+  const int ns[3] = {c->nx, c->ny, c->nz};
+  // tiling variant of the fused y/z passes (X3D_FUSED_TILING=0|1, default 0)
+  const char* tv = std::getenv("X3D_FUSED_TILING");
+  const int variant = tv ? std::atoi(tv) : 0;
+  // FP32 precision-form plans; a line they cannot tile leaves M = 0 and the
+  // FP32 step reports X3D_ERR_UNSUPPORTED
+  bool ok32 = true;
+  for (int d = 0; d < 3; ++d) ok32 = !line_plan_fused32(ns[d], d != 0, pts, &c->fplan32[d]) && ok32;
+  if (!ok32) c->fplan32[0].M = c->fplan32[1].M = c->fplan32[2].M = 0;
+  for (int d = 0; d < 3; ++d) {
+    const int rc = line_plan_fused(ns[d], d != 0, pts, &c->fplan[d], variant);
+    if (rc && !c->ncl1[d]) return rc;
+    if (rc) c->fplan[d] = LinePlan{};
+  }
+  return X3D_OK;
+}
+
 int ensure_work(x3d_ctx* c)
 {
   const size_t N = (size_t)c->nx * c->ny * c->nz;
@@ -534,31 +553,19 @@ int x3d_create_bc(int nx, int ny, int nz, double xlx, double yly, double zlz, co
     else direction_ops(c, d, ns[d]);
   }
   if (const char* xr = std::getenv("X3D_XCD_REMAP")) c->xcd_remap = std::atoi(xr) != 0;
-  // tiling variant of the fused y/z passes (X3D_FUSED_TILING=0|1, default 0)
-  const char* tv = std::getenv("X3D_FUSED_TILING");
-  const int variant = tv ? std::atoi(tv) : 0;
-  // FP32 precision-form plans; a line they cannot tile leaves M = 0 and the
-  // FP32 step reports X3D_ERR_UNSUPPORTED
-  if (line_plan_fused32(nx, false, &c->fplan32[0]) || line_plan_fused32(ny, true, &c->fplan32[1]) ||
-      line_plan_fused32(nz, true, &c->fplan32[2]))
-    c->fplan32[0].M = c->fplan32[1].M = c->fplan32[2].M = 0;
   // a non-periodic direction runs its own kernels on its own plan (lines of
   // any length); the periodic plans there may not exist, and are not used
+  const long long pts = (long long)npts;
   for (int d = 0; d < 3; ++d) {
     if (!b1[d]) continue;
     if ((rc = np_plan(ns[d], d != 0, &c->npplan[d]))) { x3d_destroy(c); return rc; }
-    if (line_plan(ns[d], d != 0, &c->plan[d])) c->plan[d] = LinePlan{};
-    if (line_plan_fused(ns[d], d != 0, &c->fplan[d], variant)) c->fplan[d] = LinePlan{};
+    if (line_plan(ns[d], d != 0, pts, &c->plan[d])) c->plan[d] = LinePlan{};
   }
   auto plans = [&]() -> int {
-    int r = X3D_OK;
-    if (!b1[0] && ((r = line_plan(nx, false, &c->plan[0])) || (r = line_plan_fused(nx, false, &c->fplan[0], variant))))
-      return r;
-    if (!b1[1] && ((r = line_plan(ny, true, &c->plan[1])) || (r = line_plan_fused(ny, true, &c->fplan[1], variant))))
-      return r;
-    if (!b1[2] && ((r = line_plan(nz, true, &c->plan[2])) || (r = line_plan_fused(nz, true, &c->fplan[2], variant))))
-      return r;
-    return r;
+    for (int d = 0; d < 3; ++d)
+      if (!b1[d])
+        if (const int r = line_plan(ns[d], d != 0, pts, &c->plan[d])) return r;
+    return fused_plans(c, pts);
   };
   if ((rc = plans()) || (rc = upload_tables(c)) || (rc = np_upload(c)) ||
       (all_periodic(c) && (rc = poisson_setup(c))) ||

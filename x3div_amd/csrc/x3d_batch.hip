@@ -188,6 +188,7 @@ std::vector<LinePlan> candidates(int n, int prec, size_t lds_max)
         if (wc * wl > 8) continue;
         LinePlan p;
         p.n = n; p.M = m; p.C = c; p.G = g; p.Wc = wc; p.Wl = wl; p.LW = 64 / g; p.line_fast = true;
+        p.bfp = p.LW % 16 == 0;
         if (plan_lds_bytes(p, prec) <= lds_max) out.push_back(p);
       }
     }
@@ -222,6 +223,12 @@ int x3d_batch_create(int ngrids, const int* dims, const double* lengths, int pre
     b->off.push_back(b->total);
     b->total += (size_t)dims[3 * i] * dims[3 * i + 1] * dims[3 * i + 2];
   }
+  // one launch covers every grid of a tiling group: tilings for the batch's points
+  for (x3d_ctx* c : b->g)
+    if (const int rc = fused_plans(c, (long long)b->total)) {
+      x3d_batch_destroy(b);
+      return rc;
+    }
   if (hipMalloc(&b->store, 10 * b->total * (size_t)precision) != hipSuccess) {
     x3d_batch_destroy(b);
     return X3D_ERR_ALLOC;

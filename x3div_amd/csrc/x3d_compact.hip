@@ -173,21 +173,94 @@ __global__ __launch_bounds__(LF ? 1024 : 256) void k_der_np(const double* in, do
 
 // Points per chunk the kernels are instantiated for.
 static const int kMs[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
+static const int kMs32[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
+template <int K>
+static bool has_chunk(const int (&ms)[K], int m)
+{
+  for (int mm : ms)
+    if (mm == m) return true;
+  return false;
+}
 
-int line_plan(int n, bool line_fast, LinePlan* P)
+// ---- line tilings ---------------------------------------------------------
+// A line is accepted when it splits into a power of two of chunks (line_plan
+// and its fused forms below); how an accepted line is cut is then chosen by
+// the chunk length, which is what a pass over lines of up to 512 points costs:
+// a solve is a serial sweep of M points and a shuffle scan over the chunks, so
+// longer chunks take fewer shuffles, halo points and wavefronts per point.
+// The chunks end where the registers of a wavefront pair do (16 FP64 or 32
+// FP32 points) or, on small grids, where too few wavefronts are left.
+// Measured, FP64 cubes, the nine passes of a step, with the shortest chunks
+// (the most per line) -> with these: 64^3 145 -> 121 us, 128^3 342 -> 238,
+// 256^3 1902 -> 1666, 320^3 4275 -> 3634; FP32 128^3 208 -> 160,
+// 320^3 2970 -> 1925.
+
+// x-lines: the longest chunk up to `cap` that leaves 8 chunks (a wavefront
+// then holds at most 8 lines; 64^3 FP64: 8 chunks of 8 points 43 us for the
+// three passes, 64 of 1 point 52).
+template <int K>
+static bool x_tiling(int n, int cap, const int (&ms)[K], LinePlan* p)
+{
+  for (int q = K - 1; q >= 0; --q) {
+    const int m = ms[q], c = n / m;
+    if (m > cap || n % m || c < 8 || c > 64 || (c & (c - 1)) || (4 + m - 1) / m > c) continue;
+    p->M = m; p->C = c; p->G = c; p->Wc = 1; p->Wl = 4; p->LW = 64 / c;
+    return true;
+  }
+  return false;
+}
+
+// y/z-lines: chunks up to `cap` points, g0 chunk groups x 64 / g0 lines per
+// wavefront (FP64 4 x 16, FP32 2 x 32: 128-byte rows), at most 8 wavefronts
+// on a line.  In this order: long chunks (3/4 of the cap or more) in a power
+// of two of whole groups, then in any number of whole groups; chunks of half
+// the cap or more, in pairs; for FP32 long chunks in any number (one group);
+// then the longest with whole groups.  (FP64 160: 10 chunks of 16 points as
+// pairs 332 us for the six y and z passes, 20 of 8 points 361; 96: 8 of 12
+// points 99 us, 32 of 3 points 155.)
+template <int K>
+static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p)
+{
+  for (int pass = 0; pass < 5; ++pass)
+    for (int q = K - 1; q >= 0; --q) {
+      const int m = ms[q], c = n / m;
+      if (m > cap || n % m || c < 4) continue;
+      int g = g0;
+      if (pass < 2 && (4 * m < 3 * cap || c % g0)) continue;
+      if (pass == 0 && (c & (c - 1))) continue;
+      if (pass == 2) {
+        if (g0 != 2 || 4 * m < 3 * cap) continue;
+        g = 1;
+      }
+      if (pass == 3) {
+        if (c % 2 || 2 * m < cap) continue;
+        g = c % g0 ? 2 : g0;
+      }
+      if (pass == 4 && c % g0) continue;
+      if (c / g > 8) continue;
+      p->M = m; p->C = c; p->G = g; p->Wc = c / g; p->Wl = 1; p->LW = 64 / g;
+      return true;
+    }
+  return false;
+}
+
+// Chunk caps by the wavefronts that the chunks leave on `pts` points: FP64 8
+// points instead of 16 below 512 wavefronts (two per compute unit); FP32 32
+// points from 1600 wavefronts on, 8 below 100.
+// (a line that 8-point chunks do not tile, 320 points, takes the longer ones)
+static bool yz_tiling64(int n, long long pts, LinePlan* p)
+{
+  return (pts / (64 * 16) < 512 && yz_tiling(n, 8, 4, kMs, p)) || yz_tiling(n, 16, 4, kMs, p);
+}
+static int yz_cap32(long long pts) { return pts / (64 * 32) >= 1600 ? 32 : (pts / (64 * 16) >= 100 ? 16 : 8); }
+
+int line_plan(int n, bool line_fast, long long pts, LinePlan* P)
 {
   if (n < 8) return X3D_ERR_SIZE;
   int C = 0, M = 0;
-  // y/z: at most 32 chunks per line first (at 512 points, 16-point chunks in
-  // 512-thread work-groups ran dery/derz 30% faster than 8-point chunks in
-  // 1024-thread ones), 64 where no shorter split exists; x: up to 64
   auto pick = [&](int cmax) {
-    for (int c = cmax; c >= 1 && !C; c >>= 1) {
-      if (n % c) continue;
-      const int m = n / c;
-      for (int mm : kMs)
-        if (mm == m) { C = c; M = m; break; }
-    }
+    for (int c = cmax; c >= 1 && !C; c >>= 1)
+      if (n % c == 0 && has_chunk(kMs, n / c)) { C = c; M = n / c; }
   };
   pick(line_fast ? 32 : 64);
   if (!C && line_fast) pick(64);
@@ -196,30 +269,33 @@ int line_plan(int n, bool line_fast, LinePlan* P)
   // of the same wavefront, at most ceil(4 / M) of them, and wrap it once
   if (!line_fast && (4 + M - 1) / M > C) return X3D_ERR_UNSUPPORTED;
   LinePlan p;
-  p.n = n; p.M = M; p.C = C; p.line_fast = line_fast;
-  if (line_fast) {
-    p.G = C < 4 ? C : 4;
-    p.Wc = C / p.G;
-    p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc;
-  } else {
-    p.G = C;
-    p.Wc = 1;
-    p.Wl = 4;
+  p.n = n; p.line_fast = line_fast;
+  if (line_fast ? !yz_tiling64(n, pts, &p) : !x_tiling(n, 8, kMs, &p)) {
+    p.M = M; p.C = C;
+    if (line_fast) {
+      p.G = C < 4 ? C : 4;
+      p.Wc = C / p.G;
+      p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc;
+    } else {
+      p.G = C;
+      p.Wc = 1;
+      p.Wl = 4;
+    }
+    p.LW = 64 / p.G;
   }
-  p.LW = 64 / p.G;
   *P = p;
   return X3D_OK;
 }
 
 // Fused passes hold several line solves per thread, so their y/z tiling caps a
-// work-group at 8 wavefronts (up to 256 VGPRs each) and takes longer chunks:
-// the largest C <= 32 chunks per line with 4 chunk groups x 16 lines per
+// work-group at 8 wavefronts (up to 256 VGPRs each): yz_tiling, else the
+// largest C <= 32 chunks per line with 4 chunk groups x 16 lines per
 // wavefront, else 64 chunks with 8 groups x 8 lines.
-int line_plan_fused(int n, bool line_fast, LinePlan* P, int variant)
+int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* P, int variant)
 {
-  if (!line_fast) return line_plan(n, false, P);
+  if (!line_fast) return line_plan(n, false, pts, P);
   if (n < 8) return X3D_ERR_SIZE;
-  auto okM = [](int m) { for (int mm : kMs) if (mm == m) return true; return false; };
+  auto okM = [](int m) { return has_chunk(kMs, m); };
   LinePlan p;
   p.n = n; p.line_fast = true;
   // explicit tiling "M,G,Wl" (chunk length, chunk groups per wavefront, line
@@ -231,6 +307,7 @@ int line_plan_fused(int n, bool line_fast, LinePlan* P, int variant)
       const int c = n / m;
       if (c <= 64 && c % g == 0 && (c / g) * wl <= 8) {
         p.C = c; p.M = m; p.G = g; p.Wc = c / g; p.Wl = wl; p.LW = 64 / g;
+        p.bfp = p.LW % 16 == 0;
         *P = p;
         return X3D_OK;
       }
@@ -246,33 +323,38 @@ int line_plan_fused(int n, bool line_fast, LinePlan* P, int variant)
     if (n % c || !okM(n / c)) continue;
     p.C = c; p.M = n / c; p.G = c < 4 ? c : 4; p.Wc = c / p.G;
     p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc; p.LW = 64 / p.G;
+    (void)yz_tiling64(n, pts, &p);
+    p.bfp = p.LW % 16 == 0;
     *P = p;
     return X3D_OK;
   }
   if (n % 64 == 0 && okM(n / 64)) {
     p.C = 64; p.M = n / 64; p.G = 8; p.Wc = 8; p.Wl = 1; p.LW = 8;
+    (void)yz_tiling64(n, pts, &p);
     *P = p;
     return X3D_OK;
   }
   return X3D_ERR_UNSUPPORTED;
 }
 
-// FP32 fused y/z passes: the same scheme with chunks up to 32 points, tiled
-// for 128-byte rows where the line allows (32 lines x 2 chunk groups per
+// FP32 fused passes: x chunks up to 16 points, y/z chunks up to 32, tiled for
+// 128-byte rows where the line allows (32 lines x 2 chunk groups per
 // wavefront), else 16 x 4 or 8 x 8; at most 8 wavefronts per work-group.
-static const int kMs32[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
-
-int line_plan_fused32(int n, bool line_fast, LinePlan* P)
+int line_plan_fused32(int n, bool line_fast, long long pts, LinePlan* P)
 {
-  if (!line_fast) return line_plan(n, false, P);
+  if (!line_fast) {
+    const int rc = line_plan(n, false, pts, P);
+    if (!rc) (void)x_tiling(n, 16, kMs, P);
+    return rc;
+  }
   if (n < 8) return X3D_ERR_SIZE;
-  auto okM = [](int m) { for (int mm : kMs32) if (mm == m) return true; return false; };
   for (int g : {2, 4, 8}) {
     for (int c = 8 * g; c >= g; c >>= 1) {
-      if (n % c || !okM(n / c)) continue;
+      if (n % c || !has_chunk(kMs32, n / c)) continue;
       LinePlan p;
       p.n = n; p.line_fast = true; p.C = c; p.M = n / c; p.G = g; p.Wc = c / g; p.LW = 64 / g;
       p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc;
+      (void)yz_tiling(n, yz_cap32(pts), 2, kMs32, &p);
       *P = p;
       return X3D_OK;
     }

@@ -588,13 +588,14 @@ static DirSet<S> dirset(const x3d_ctx* c, int dir)
   } while (0)
 
 // BFP32 fields: a y/z-line lane group must be 16 lines (one x-segment) or a
-// multiple, and x rows whole segments.
+// multiple, and x rows whole segments.  Lines that only 64 chunks split into a
+// power of two (320, 768, 1024 points) are not taken.
 template <typename S>
 static bool storage_ok(const x3d_ctx* c, int dir)
 {
   if constexpr (!is_bfp<S>) return true;
   const LinePlan& P = fused_plan<S>(c, dir);
-  return c->nx % 16 == 0 && (!P.line_fast || P.LW % 16 == 0);
+  return c->nx % 16 == 0 && (!P.line_fast || P.bfp);
 }
 
 template <int DIR, typename S>

@@ -65,6 +65,7 @@ struct LinePlan {
   int Wl = 0;     // independent line groups per work-group
   int LW = 0;     // lines per wavefront (64 / G)
   bool line_fast = false;  // lanes: consecutive lines (y/z) or consecutive chunks (x)
+  bool bfp = false;  // fused y/z: the BFP32 step takes the line (one of at most 32 chunks, whole 16-line rows)
 };
 
 }  // namespace x3d
@@ -214,8 +215,9 @@ constexpr bool transeq_zfirst() { return !std::is_same<S, float>::value; }
 // stream for theirs (join; also after an error, returning the first one).
 int batch_fork(x3d_batch* b);
 int batch_join(x3d_batch* b, int rc);
-int line_plan(int n, bool line_fast, LinePlan* out);
-int line_plan_fused(int n, bool line_fast, LinePlan* out, int variant);
+// Line tilings for lines of n points; pts: the points one launch covers.
+int line_plan(int n, bool line_fast, long long pts, LinePlan* out);
+int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* out, int variant);
 
 // Launch one compact operator (or Thomas alone) along direction dir.
 int launch_line_f32(x3d_ctx* c, int dir, int kind, int op, const float* in, float* out);
@@ -274,7 +276,10 @@ void launch_dims(const x3d_ctx* c, int dir, Geom* geo, Tiling* tl, dim3* grid, d
                  size_t tbytes, bool fused = false);
 void launch_dims_plan(const x3d_ctx* c, int dir, const LinePlan& P, Geom* geo, Tiling* tl, dim3* grid,
                       dim3* block, size_t* smem, size_t tbytes);
-int line_plan_fused32(int n, bool line_fast, LinePlan* out);
+int line_plan_fused32(int n, bool line_fast, long long pts, LinePlan* out);
+// The fused plans of a context, FP64 and FP32, for launches of pts points (its
+// own, or those of the batch it belongs to).
+int fused_plans(x3d_ctx* c, long long pts);
 
 int poisson_setup(x3d_ctx* c);
 void poisson_release(x3d_ctx* c);
