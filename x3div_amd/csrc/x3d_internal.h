@@ -117,6 +117,7 @@ struct x3d_ctx {
   bool timing = false;
   // dense-circulant fragments of the matrix-core variant, per operator (made on first use)
   void* circ_tab[X3D_NOPS] = {};
+  int circ_lo[X3D_NOPS] = {}, circ_count[X3D_NOPS] = {};  // block offsets each table holds
   float circ_scale[X3D_NOPS] = {};  // 2^-s of the power-of-two scaling of each table
   // captured step (x3d_graph_capture_step*, or the calls between
   // x3d_graph_begin and x3d_graph_end), replayed by x3d_graph_launch
