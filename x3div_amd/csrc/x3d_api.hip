@@ -1096,10 +1096,10 @@ int x3d_step(x3d_ctx* c, double gdt, double* ux, double* uy, double* uz, double*
     X3D_TRY(x3d_cor_vel(c, ux, uy, uz, px, py, pz));
     return X3D_OK;
   }
-  // transeq with the Euler update folded into its x pass, divergence, Poisson,
-  // gradp with cor_vel folded into its x pass
-  X3D_TRY(fused_momentum<double>(c, gdt, 1, ux, uy, uz, dux, duy, duz));
-  X3D_TRY(fused_divergence<double>(c, pp3, ux, uy, uz));
+  // transeq with the Euler update and the divergence's x operators folded into
+  // its x pass, the rest of the divergence, Poisson, gradp with cor_vel folded
+  // into its x pass
+  X3D_TRY(fused_momentum_divergence<double>(c, gdt, ux, uy, uz, dux, duy, duz, pp3));
   X3D_TRY(poisson_solve(c, pp3));
   X3D_TRY(mark_pass(c, 7));
   X3D_TRY(fused_gradp<double>(c, px, py, pz, pp3, ux, uy, uz, 1));
@@ -1172,8 +1172,7 @@ int x3d_step_f32(x3d_ctx* c, double gdt, float* ux, float* uy, float* uz, float*
   if (!c || !ux || !uy || !uz || !dux || !duy || !duz || !pp3 || !px || !py || !pz) return X3D_ERR_ARG;
   if (!all_periodic(c)) return X3D_ERR_UNSUPPORTED;
   if (!fp32_ok(c)) return X3D_ERR_UNSUPPORTED;
-  X3D_TRY(fused_momentum<float>(c, (float)gdt, 1, ux, uy, uz, dux, duy, duz));
-  X3D_TRY(fused_divergence<float>(c, pp3, ux, uy, uz));
+  X3D_TRY(fused_momentum_divergence<float>(c, (float)gdt, ux, uy, uz, dux, duy, duz, pp3));
   X3D_TRY(poisson_solve_f32(c, pp3));
   X3D_TRY(mark_pass(c, 7));
   X3D_TRY(fused_gradp<float>(c, px, py, pz, pp3, ux, uy, uz, 1));
@@ -1195,8 +1194,6 @@ int x3d_step_timed_f32(x3d_ctx* c, double gdt, float* ux, float* uy, float* uz, 
   X3D_CHECK_HIP(hipEventSynchronize(c->pass_ev[X3D_NPASS]));
   for (int i = 0; i < X3D_NPASS; ++i)
     X3D_CHECK_HIP(hipEventElapsedTime(&pass_ms[i], c->pass_ev[i], c->pass_ev[i + 1]));
-  // the pass names follow the z-first transeq order
-  if (!transeq_zfirst<float>()) std::swap(pass_ms[0], pass_ms[2]);
   return X3D_OK;
 }
 

@@ -17,18 +17,14 @@
 namespace x3d {
 
 // ---- transeq: r_c = D(u_d u_c) + u_d D(u_c), d = DIR ----------------------
-// ZF (z first): Z: du_c = r_c; Y: tmp_c = du_c + r_c;
-//               X: du_c = tmp_c + r_c; if euler: u_c = gdt du_c + u_c.
-// else:         X: du_c = r_c; Y: tmp_c = du_c + r_c;
-//               Z: du_c = tmp_c + r_c; if euler: u_c = gdt du_c + u_c.
+// Z: du_c = r_c; Y: tmp_c = du_c + r_c;
+// X: du_c = tmp_c + r_c; if euler: u_c = gdt du_c + u_c.
 // (src/transeq.f90:100-115, 120-134, 139-153, 158-177 per component; the
-// reference sums the x, y, z parts in that order, ZF the z, y, x parts: the
-// same terms, rounded in another order.)  With ZF the z pass, whose strided
-// rows cost an address translation each, reads u and writes one part (6
-// fields), and the x pass, whose rows are contiguous, carries the sums and
-// the Euler update (12 fields).  Measured at 512^3, that is faster for FP64
-// (6.81 -> 6.75 ms for the three passes) and BFP32 (6.81 -> 5.86 ms), slower
-// for FP32 (3.11 -> 3.21 ms), whose single grids keep x first.
+// reference sums the x, y, z parts in that order, here the z, y, x parts: the
+// same terms, rounded in another order.)  The z pass, whose strided rows cost
+// an address translation each, reads u and writes one part (6 fields), and the
+// x pass, whose rows are contiguous, carries the sums and the Euler update (12
+// fields), and in a step the divergence's x operators.
 // S: the fields' storage (FP64, FP32, or BFP32 computed in FP64).
 template <typename S>
 struct TranseqArgs {
@@ -43,12 +39,27 @@ struct TranseqArgs {
   const T* sy;  // y-stretching ppy(j), or nullptr (y pass only)
 };
 
-template <typename S, int M, int DIR, bool ZF>
-__device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ A, int blk)
+// The divergence's x operators, applied by the last x pass of a step to the
+// velocities that it has just updated: o1 = Dvp(ux), o2 = Ivp(uy), o3 = Ivp(uz).
+template <typename S>
+struct DivXArgs {
+  using T = typename Store<S>::T;
+  S *o1, *o2, *o3;
+  Coef<T> cfd;
+  Circ<T> ccd;
+  Coef<T> cfi;
+  Circ<T> cci;
+};
+
+// DX (last x pass of a step): each updated u_c is in the staging tile when it
+// has been stored, so the x operators of the divergence, whose lines are the
+// same, take it from there: the pass writes their three results (15 fields
+// with the rest) and the divergence's own x pass, which would read u again (6
+// fields), falls away.  What bounds it is HBM, 15 fields at the copy rate.
+template <typename S, int M, int DIR, bool DX = false>
+__device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ A, int blk,
+                                             const DivXArgs<S>* __restrict__ X = nullptr)
 {
-  // this pass's place in the order: the first writes du_c, the last adds
-  // tmp_c and applies the Euler update
-  constexpr bool FIRST = DIR == (ZF ? 2 : 0), LAST = DIR == (ZF ? 0 : 2);
   using T = typename Store<S>::T;
   S* const ux = A.ux; S* const uy = A.uy; S* const uz = A.uz;
   S* const dux = A.dux; S* const duy = A.duy; S* const duz = A.duz;
@@ -72,20 +83,20 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
     xd = x_block<S, M>(geo, t, lds + (blockDim.x >> 6) * x_tile_words<M>());
     x_stage_in<S, M>(Ud, xd);
   }
-  // y/z: the u_d window (the same for the three components) and, for the
-  // Euler update of a last z pass, each u_c chunk are kept in per-thread LDS
-  // slots from their loads to their later uses instead of being loaded again:
-  // strided loads cost address translation per row, LDS slots do not.  Slot
-  // q of thread i is keep[q * blockDim.x + i], after the solver's words.
+  // y/z: the u_d window (the same for the three components) is kept in
+  // per-thread LDS slots from its load to its later uses instead of being
+  // loaded again: strided loads cost address translation per row, LDS slots do
+  // not.  Slot q of thread i is keep[q * blockDim.x + i], after the solver's
+  // words.
   T* const keep = lds + line_lds_words(t.Wc, t.LPW);
   const int nth = blockDim.x, tid = threadIdx.x;
-  // a first z pass: the u_y window of the second component is loaded during
+  // z: the u_y window of the second component is loaded during
   // the first component's line solves (its strided rows wait on address
   // translation) and formed when it is used.  FP64 arithmetic (FP64 and
   // BFP32 fields) with 16-point chunks only, whose 512-thread work-groups
   // hold 2 waves per SIMD with or without the window's registers (shorter
   // chunks would lose occupancy).
-  constexpr bool PREW = DIR == 2 && FIRST && sizeof(T) == 8 && M >= 16;
+  constexpr bool PREW = DIR == 2 && sizeof(T) == 8 && M >= 16;
   RawT<S> pw[PREW ? NW : 1];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -130,10 +141,6 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
           }
           if (!formed) load_window<S, M, H, H, true>(Uc, t, n, wc);
         }
-        if constexpr (DIR == 2 && LAST) {
-#pragma unroll
-          for (int k = 0; k < M; ++k) keep[(NW + k) * nth + tid] = wc[H + k];
-        }
       }
       rhs_chunk<K_D, T, M, H>(wc, cf, v2);
 #pragma unroll
@@ -143,26 +150,24 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
                 cf.b * (wd[q + 2] * wc[q + 2] - wd[q - 2] * wc[q - 2]);
       }
     }
-    // y, and a last z pass: the epilogue's strided loads (du_c of the first
-    // pass, resp. tmp_c) are issued here and complete during the two line
-    // solves, whose barriers wait on LDS only.  Neither field is written by
-    // this pass.  (not for FP32 z-lines of 32-point chunks, which would spill)
-    constexpr bool PF = DIR == 1 || (DIR == 2 && LAST && !(sizeof(T) == 4 && M >= 32));
+    // y: the epilogue's strided loads (du_c of the z pass) are issued here and
+    // complete during the two line solves, whose barriers wait on LDS only.
+    // The field is not written by this pass.
+    constexpr bool PF = DIR == 1;
     if constexpr (PREW) {
       if (c == 0) window_issue<S, M, H, H>(uy, t, n, pw);
     }
-    // a last x pass in FP64: the coalesced loads of tmp_c likewise (measured:
+    // x in FP64: the coalesced loads of tmp_c likewise (measured:
     // FP64 512^3 2.45 -> 2.42 ms; the FP32 batch lost a wave and ran slower)
-    constexpr bool PFX = DIR == 0 && LAST && M % 2 == 0 && !is_bfp<S> && sizeof(T) == 8;
+    constexpr bool PFX = DIR == 0 && M % 2 == 0 && !is_bfp<S> && sizeof(T) == 8;
     // (storage words, decoded at use: a BFP32 decode would wait for them here)
     T a[M];
     RawT<S> ar[M];
     if constexpr (PFX) x_fetch<S, M>(TMc, xb, a);
     if constexpr (PF) {
       if (t.active) {
-        const S* src = DIR == 1 ? DUc : TMc;  // (DIR 2: tmp_c)
 #pragma unroll
-        for (int k = 0; k < M; ++k) ar[k] = ld_raw(src, t.at(t.j0 + k));
+        for (int k = 0; k < M; ++k) ar[k] = ld_raw(DUc, t.at(t.j0 + k));
       }
     }
     // keep the two line solves apart: interleaving them doubles the live state
@@ -180,9 +185,7 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
 #pragma unroll
       for (int k = 0; k < M; ++k) v1[k] = v1[k] + keep[(H + k) * nth + tid] * v2[k];
     }
-    if constexpr (DIR == 0 && FIRST) {
-      x_store<S, M>(DUc, xb, v1);
-    } else if constexpr (DIR == 0) {
+    if constexpr (DIR == 0) {
       // du_c = tmp_c + r_c and the Euler update, through the staging tile:
       // u_c at the chunk points first (the u_x tile, resp. the tile still
       // holding this component's window load), then tmp_c restaged (its
@@ -208,6 +211,20 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
 #pragma unroll
         for (int k = 0; k < M; ++k) v1[k] = gdt * v1[k] + uc[k];
         x_store<S, M>(Uc, xb, v1);
+        if constexpr (DX) {
+          if (c == 0) {
+            T w[M + 3];
+            x_window<S, M, 1, 2>(xb, t, w);
+            rhs_chunk<K_DVP, T, M, 1>(w, X->cfd, v1);
+            solve_circ<T, M, false>(v1, t, X->ccd, lds);
+          } else {
+            T w[M + 7];
+            x_window<S, M, 3, 4>(xb, t, w);
+            rhs_chunk<K_IVP, T, M, 3>(w, X->cfi, v1);
+            solve_circ<T, M, false>(v1, t, X->cci, lds);
+          }
+          x_store<S, M>(c == 0 ? X->o1 : (c == 1 ? X->o2 : X->o3), xb, v1);
+        }
       }
     } else if constexpr (DIR == 1) {
       // tmp_c = du_c (first pass's part) + r_c: the sum is formed here, where
@@ -220,27 +237,10 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
 #pragma unroll
         for (int k = 0; k < M; ++k) sst(TMc, t.at(t.j0 + k), from_raw<S>(ar[k]) + v1[k]);
       }
-    } else if constexpr (FIRST) {
+    } else {
       if (t.active) {
 #pragma unroll
         for (int k = 0; k < M; ++k) sst(DUc, t.at(t.j0 + k), v1[k]);
-      }
-    } else {
-      if (t.active) {
-        if constexpr (PF) {
-#pragma unroll
-          for (int k = 0; k < M; ++k) a[k] = from_raw<S>(ar[k]);
-        } else {
-#pragma unroll
-          for (int k = 0; k < M; ++k) a[k] = sld(TMc, t.at(t.j0 + k));
-        }
-#pragma unroll
-        for (int k = 0; k < M; ++k) {
-          const uint32_t at = t.at(t.j0 + k);
-          const T d = a[k] + v1[k];
-          sst(DUc, at, d);
-          if (euler) sst(Uc, at, gdt * d + keep[(NW + k) * nth + tid]);
-        }
       }
     }
   }
@@ -445,8 +445,14 @@ __device__ __forceinline__ int grid_of(const int* __restrict__ block0, int ngrid
   return lo;
 }
 
-template <typename S, int M, int DIR, bool ZF>
-__global__ __launch_bounds__(512) void k_transeq(TranseqArgs<S> A) { transeq_body<S, M, DIR, ZF>(A, A.tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x); }
+template <typename S, int M, int DIR>
+__global__ __launch_bounds__(512) void k_transeq(TranseqArgs<S> A) { transeq_body<S, M, DIR>(A, A.tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x); }
+// (held to the registers of the pass without the divergence: FP64 chunks of 8
+// points would take 131 and leave 3 wavefronts per SIMD, of 12 points 172 and 2)
+template <typename S, int M>
+constexpr int divx_waves() { return sizeof(S) == 8 ? (M <= 8 ? 4 : M <= 12 ? 3 : 1) : 1; }
+template <typename S, int M>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(divx_waves<S, M>()))) void k_transeq_div_x(TranseqArgs<S> A, DivXArgs<S> X) { transeq_body<S, M, 0, true>(A, blockIdx.x, &X); }
 // y passes: at most 128 VGPRs, so that two work-groups share a compute unit
 // (measured faster at 512^3 in both precisions despite a few spills)
 template <typename S, int M, int DIR>
@@ -461,7 +467,18 @@ __global__ __launch_bounds__(512) void k_transeq_batch(const TranseqArgs<T>* __r
   const int total = block0[ngrids];
   for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
     const int g = grid_of(block0, ngrids, vb);
-    transeq_body<T, M, DIR, true>(list[g], vb - block0[g]);
+    transeq_body<T, M, DIR>(list[g], vb - block0[g]);
+  }
+}
+template <typename T, int M>
+__global__ __launch_bounds__(512) void k_transeq_div_x_batch(const TranseqArgs<T>* __restrict__ list,
+                                                             const DivXArgs<T>* __restrict__ xlist,
+                                                             const int* __restrict__ block0, int ngrids)
+{
+  const int total = block0[ngrids];
+  for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
+    const int g = grid_of(block0, ngrids, vb);
+    transeq_body<T, M, 0, true>(list[g], vb - block0[g], xlist + g);
   }
 }
 template <typename T, int M, int DIR>
@@ -608,12 +625,33 @@ static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz,
   const TranseqArgs<S> A{ux,   uy,   uz,   dux,  duy,      duz,   tx,
                          ty,   tz,   s.cf_d, s.cc_d, s.geo, s.tl, (T)gdt,
                          euler, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
-  // (a last z pass keeps each u_c chunk for the Euler update as well)
-  constexpr bool ZF = transeq_zfirst<S>();
-  const size_t smem = s.smem_tq + (DIR == 2 && !ZF ? sizeof(T) * (size_t)s.block.x * (size_t)s.M : 0);
   X3D_MSWITCH_T(S, s.M, {
-    allow_lds((const void*)k_transeq<S, MM, DIR, ZF>, smem);
-    hipLaunchKernelGGL((k_transeq<S, MM, DIR, ZF>), s.grid, s.block, smem, c->stream, A);
+    allow_lds((const void*)k_transeq<S, MM, DIR>, s.smem_tq);
+    hipLaunchKernelGGL((k_transeq<S, MM, DIR>), s.grid, s.block, s.smem_tq, c->stream, A);
+  });
+  X3D_CHECK_HIP(hipGetLastError());
+  return X3D_OK;
+}
+
+// The last transeq pass of a step, with the divergence's x operators.
+template <typename S>
+static DivXArgs<S> divx_args(const DirSet<S>& s, S* o1, S* o2, S* o3)
+{
+  return DivXArgs<S>{o1, o2, o3, s.cf_dvp, s.cc_s, s.cf_ivp, s.cc_i};
+}
+
+template <typename S>
+static int transeq_div_x_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz, S* tx, S* ty, S* tz, double gdt,
+                              S* o1, S* o2, S* o3)
+{
+  using T = typename Store<S>::T;
+  if (!storage_ok<S>(c, 0)) return X3D_ERR_UNSUPPORTED;
+  const DirSet<S> s = dirset<S>(c, 0);
+  const TranseqArgs<S> A{ux, uy, uz, dux, duy, duz, tx, ty, tz, s.cf_d, s.cc_d, s.geo, s.tl, (T)gdt, 1, nullptr};
+  const DivXArgs<S> X = divx_args(s, o1, o2, o3);
+  X3D_MSWITCH_T(S, s.M, {
+    allow_lds((const void*)k_transeq_div_x<S, MM>, s.smem_tq);
+    hipLaunchKernelGGL((k_transeq_div_x<S, MM>), s.grid, s.block, s.smem_tq, c->stream, A, X);
   });
   X3D_CHECK_HIP(hipGetLastError());
   return X3D_OK;
@@ -666,13 +704,25 @@ int fused_momentum(x3d_ctx* c, double gdt, int euler, T* ux, T* uy, T* uz, T* du
   if (sizeof(T) == 8 && !c->f64_lines) return X3D_ERR_UNSUPPORTED;
   X3D_TRY(ensure_work(c));
   T *tx = wk<T>(c, 5), *ty = wk<T>(c, 6), *tz = wk<T>(c, 7);
-  constexpr int D0 = transeq_zfirst<T>() ? 2 : 0;  // first pass; the last is 2 - D0
-  X3D_TRY((transeq_pass<D0, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+  X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
   X3D_TRY(mark_pass(c, 1));
   X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
   X3D_TRY(mark_pass(c, 2));
-  X3D_TRY((transeq_pass<2 - D0, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, euler)));
+  X3D_TRY((transeq_pass<0, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, euler)));
   X3D_TRY(mark_pass(c, 3));
+  return X3D_OK;
+}
+
+// The divergence's y and z passes, from the results of its x pass in the work
+// fields 0-2.
+template <typename T>
+static int divergence_yz(x3d_ctx* c, T* pp3)
+{
+  T *pp1 = wk<T>(c, 0), *pgy1 = wk<T>(c, 1), *pgz1 = wk<T>(c, 2), *dd2 = wk<T>(c, 3), *upi2 = wk<T>(c, 4);
+  X3D_TRY((div_pass<1, T>(c, pp1, pgy1, pgz1, dd2, upi2, nullptr)));
+  X3D_TRY(mark_pass(c, 5));
+  X3D_TRY((div_pass<2, T>(c, dd2, upi2, nullptr, pp3, nullptr, nullptr)));
+  X3D_TRY(mark_pass(c, 6));
   return X3D_OK;
 }
 
@@ -681,14 +731,34 @@ int fused_divergence(x3d_ctx* c, T* pp3, const T* ux, const T* uy, const T* uz)
 {
   if (sizeof(T) == 8 && !c->f64_lines) return X3D_ERR_UNSUPPORTED;
   X3D_TRY(ensure_work(c));
-  T *pp1 = wk<T>(c, 0), *pgy1 = wk<T>(c, 1), *pgz1 = wk<T>(c, 2), *dd2 = wk<T>(c, 3), *upi2 = wk<T>(c, 4);
-  X3D_TRY((div_pass<0, T>(c, ux, uy, uz, pp1, pgy1, pgz1)));
+  X3D_TRY((div_pass<0, T>(c, ux, uy, uz, wk<T>(c, 0), wk<T>(c, 1), wk<T>(c, 2))));
   X3D_TRY(mark_pass(c, 4));
-  X3D_TRY((div_pass<1, T>(c, pp1, pgy1, pgz1, dd2, upi2, nullptr)));
-  X3D_TRY(mark_pass(c, 5));
-  X3D_TRY((div_pass<2, T>(c, dd2, upi2, nullptr, pp3, nullptr, nullptr)));
-  X3D_TRY(mark_pass(c, 6));
-  return X3D_OK;
+  return divergence_yz<T>(c, pp3);
+}
+
+// Momentum with the Euler update, then the divergence, as the step runs them:
+// the divergence's x operators ride in the last transeq pass (512^3: FP64 3.55
+// -> 3.04 ms for the two, FP32 1.82 -> 1.51).  BFP32 keeps two passes: its x
+// passes are bound by the coder's instructions, and the fused one would code
+// u twice (2.53 -> 2.73 ms).  So does the per-pass timing (the same operations
+// on the same values), so that each pass has a time of its own.
+template <typename T>
+int fused_momentum_divergence(x3d_ctx* c, double gdt, T* ux, T* uy, T* uz, T* dux, T* duy, T* duz, T* pp3)
+{
+  if (is_bfp<T> || c->timing) {
+    X3D_TRY(fused_momentum<T>(c, gdt, 1, ux, uy, uz, dux, duy, duz));
+    return fused_divergence<T>(c, pp3, ux, uy, uz);
+  }
+  if constexpr (!is_bfp<T>) {
+    if (sizeof(T) == 8 && !c->f64_lines) return X3D_ERR_UNSUPPORTED;
+    X3D_TRY(ensure_work(c));
+    T *tx = wk<T>(c, 5), *ty = wk<T>(c, 6), *tz = wk<T>(c, 7);
+    X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+    X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+    X3D_TRY((transeq_div_x_pass<T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, wk<T>(c, 0), wk<T>(c, 1),
+                                   wk<T>(c, 2))));
+  }
+  return divergence_yz<T>(c, pp3);
 }
 
 template <typename T>
@@ -716,6 +786,8 @@ struct PlanKey {
   }
 };
 constexpr int kPassDir[9] = {2, 1, 0, 0, 1, 2, 2, 1, 0};
+// (pass 3, the divergence along x, rides in pass 2)
+constexpr int kDivX = 3;
 }  // namespace
 
 template <typename T>
@@ -735,6 +807,7 @@ int batch_build(x3d_batch* b, double gdt)
   b->launches.clear();
   for (int i = 0; i < b->ng; ++i) X3D_TRY(ensure_work(b->g[i]));
   for (int pass = 0; pass < 9; ++pass) {
+    if (pass == kDivX) continue;
     const int dir = kPassDir[pass];
     std::map<PlanKey, std::vector<int>> groups;
     for (int i = 0; i < b->ng; ++i) {
@@ -748,6 +821,7 @@ int batch_build(x3d_batch* b, double gdt)
       L.pass = pass;
       L.M = kv.first.M;
       std::vector<TranseqArgs<T>> ta;
+      std::vector<DivXArgs<T>> xa;
       std::vector<PassArgs<T>> pa;
       for (int i : kv.second) {
         x3d_ctx* c = b->g[i];
@@ -759,10 +833,10 @@ int batch_build(x3d_batch* b, double gdt)
         if (pass < 3) {
           ta.push_back(TranseqArgs<T>{f[0], f[1], f[2], f[3], f[4], f[5], w[5], w[6], w[7], s.cf_d, s.cc_d, s.geo,
                                       s.tl, (T)gdt, pass == 2 ? 1 : 0});
+          if (pass == 2) xa.push_back(divx_args<T>(s, w[0], w[1], w[2]));
         } else if (pass < 6) {
           const T *a = nullptr, *bb = nullptr, *cc = nullptr;
           T *o1 = nullptr, *o2 = nullptr, *o3 = nullptr;
-          if (pass == 3) { a = f[0]; bb = f[1]; cc = f[2]; o1 = w[0]; o2 = w[1]; o3 = w[2]; }
           if (pass == 4) { a = w[0]; bb = w[1]; cc = w[2]; o1 = w[3]; o2 = w[4]; }
           if (pass == 5) { a = w[3]; bb = w[4]; o1 = f[6]; }
           pa.push_back(PassArgs<T>{a, bb, cc, o1, o2, o3, nullptr, nullptr, nullptr, s.cf_dvp, s.cc_s, s.cf_ivp,
@@ -783,6 +857,7 @@ int batch_build(x3d_batch* b, double gdt)
       L.ngroup = (int)kv.second.size();
       L.args = pass < 3 ? put(ta.data(), ta.size() * sizeof(TranseqArgs<T>))
                         : put(pa.data(), pa.size() * sizeof(PassArgs<T>));
+      if (pass == 2) L.xargs = put(xa.data(), xa.size() * sizeof(DivXArgs<T>));
       L.block0 = put(block0.data(), block0.size() * sizeof(int));
       // persistent: at most a few work-groups per compute unit walk the blocks
       const int cap = 4 * b->ncu;
@@ -819,8 +894,15 @@ static int batch_launch(x3d_batch* b, const x3d_batch::Launch& L, hipStream_t st
       hipLaunchKernelGGL((K<T, MM, DIR>), L.grid, L.block, L.smem, st, LIST, block0, L.ngroup);           \
     });                                                                                                   \
     break;
-    X3D_BT(0, k_transeq_batch, 2, ta) X3D_BT(1, k_transeq_batch, 1, ta) X3D_BT(2, k_transeq_batch, 0, ta)
-    X3D_BT(3, k_div_batch, 0, pa) X3D_BT(4, k_div_batch, 1, pa) X3D_BT(5, k_div_batch, 2, pa)
+    X3D_BT(0, k_transeq_batch, 2, ta) X3D_BT(1, k_transeq_batch, 1, ta)
+    case 2:
+      X3D_MSWITCH_T(T, L.M, {
+        allow_lds((const void*)k_transeq_div_x_batch<T, MM>, L.smem);
+        hipLaunchKernelGGL((k_transeq_div_x_batch<T, MM>), L.grid, L.block, L.smem, st, ta,
+                           reinterpret_cast<const DivXArgs<T>*>(base + L.xargs), block0, L.ngroup);
+      });
+      break;
+    X3D_BT(4, k_div_batch, 1, pa) X3D_BT(5, k_div_batch, 2, pa)
     X3D_BT(6, k_grad_batch, 2, pa) X3D_BT(7, k_grad_batch, 1, pa) X3D_BT(8, k_grad_batch, 0, pa)
 #undef X3D_BT
     default: return X3D_ERR_ARG;
@@ -860,6 +942,11 @@ template int batch_passes<float>(x3d_batch*, int);
 template int fused_momentum<double>(x3d_ctx*, double, int, double*, double*, double*, double*, double*, double*);
 template int fused_momentum<float>(x3d_ctx*, double, int, float*, float*, float*, float*, float*, float*);
 template int fused_momentum<bfp32>(x3d_ctx*, double, int, bfp32*, bfp32*, bfp32*, bfp32*, bfp32*, bfp32*);
+template int fused_momentum_divergence<double>(x3d_ctx*, double, double*, double*, double*, double*, double*, double*,
+                                               double*);
+template int fused_momentum_divergence<float>(x3d_ctx*, double, float*, float*, float*, float*, float*, float*, float*);
+template int fused_momentum_divergence<bfp32>(x3d_ctx*, double, bfp32*, bfp32*, bfp32*, bfp32*, bfp32*, bfp32*,
+                                              bfp32*);
 template int fused_divergence<double>(x3d_ctx*, double*, const double*, const double*, const double*);
 template int fused_divergence<float>(x3d_ctx*, float*, const float*, const float*, const float*);
 template int fused_divergence<bfp32>(x3d_ctx*, bfp32*, const bfp32*, const bfp32*, const bfp32*);

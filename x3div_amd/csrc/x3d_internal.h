@@ -152,11 +152,12 @@ struct x3d_batch {
   // device argument records of the grouped launches, rebuilt when the plans
   // or gdt change
   struct Launch {
-    int pass;       // 0-2 transeq z y x, 3-5 divergence x y z, 6-8 gradp z y x
+    int pass;       // 0-2 transeq z y x (2 with divergence x), 4-5 divergence y z, 6-8 gradp z y x
     int M;
     dim3 grid, block;
     size_t smem;
     size_t args;    // byte offset of the group's records in dargs
+    size_t xargs;   // pass 2: and of its divergence-x records
     size_t block0;  // byte offset of its block prefix (ngroup + 1 ints)
     int ngroup;
   };
@@ -207,11 +208,6 @@ template <typename T>
 int batch_build(x3d_batch* b, double gdt);
 template <typename T>
 int batch_passes(x3d_batch* b, int which);
-// Order of the single-grid transeq passes for storage S: z, y, x (true), or
-// x, y, z for FP32 (measured faster there).  The batch always runs z, y, x.
-// The timed steps report the passes under the names of the z-first order.
-template <typename S>
-constexpr bool transeq_zfirst() { return !std::is_same<S, float>::value; }
 // The side streams wait for the batch stream's work so far (fork), the batch
 // stream for theirs (join; also after an error, returning the first one).
 int batch_fork(x3d_batch* b);
@@ -318,6 +314,8 @@ inline bool all_periodic(const x3d_ctx* c)
 bool fused_ok(const x3d_ctx* c);
 template <typename T>
 int fused_momentum(x3d_ctx* c, double gdt, int euler, T* ux, T* uy, T* uz, T* dux, T* duy, T* duz);
+template <typename T>
+int fused_momentum_divergence(x3d_ctx* c, double gdt, T* ux, T* uy, T* uz, T* dux, T* duy, T* duz, T* pp3);
 template <typename T>
 int fused_divergence(x3d_ctx* c, T* pp3, const T* ux, const T* uy, const T* uz);
 template <typename T>
