@@ -611,11 +611,7 @@ int x3d_set_stream(x3d_ctx* c, void* stream)
 {
   if (!c) return X3D_ERR_ARG;
   c->stream = (hipStream_t)stream;
-  if (c->fft_ready) {
-    if (hipfftSetStream(c->fft_r2c, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
-    if (hipfftSetStream(c->fft_c2r, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
-  }
-  return X3D_OK;
+  return fft_streams(c, c->stream);
 }
 
 int x3d_sync(x3d_ctx* c)
@@ -1204,17 +1200,6 @@ static void graph_release(x3d_ctx* c)
   if (c->graph) (void)hipGraphDestroy(c->graph);
   c->graph_exec = nullptr;
   c->graph = nullptr;
-}
-
-static int fft_streams(x3d_ctx* c, hipStream_t s)
-{
-  if (c->fft_ready && (hipfftSetStream(c->fft_r2c, s) != HIPFFT_SUCCESS ||
-                       hipfftSetStream(c->fft_c2r, s) != HIPFFT_SUCCESS))
-    return X3D_ERR_FFT;
-  if (c->fft32_ready && (hipfftSetStream(c->fft_r2c32, s) != HIPFFT_SUCCESS ||
-                         hipfftSetStream(c->fft_c2r32, s) != HIPFFT_SUCCESS))
-    return X3D_ERR_FFT;
-  return X3D_OK;
 }
 
 // Record body's launches on a private stream into a graph; every allocation

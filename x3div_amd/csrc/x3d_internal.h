@@ -279,6 +279,8 @@ int line_plan_fused32(int n, bool line_fast, long long pts, LinePlan* out);
 int fused_plans(x3d_ctx* c, long long pts);
 
 int poisson_setup(x3d_ctx* c);
+// every FFT plan of the context onto stream s
+int fft_streams(x3d_ctx* c, hipStream_t s);
 void poisson_release(x3d_ctx* c);
 int poisson_solve(x3d_ctx* c, double* rhs);
 // BFP32 right-hand side, solved in FP64 and stored back as BFP32 words, the

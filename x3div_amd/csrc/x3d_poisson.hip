@@ -1232,9 +1232,16 @@ static int twiddles(int n, void** dev)
 // r2c into one pass there, while its 1-D batched r2c takes two), else the
 // whole 3-D transform.  Inverse: the x c2r of every row when the y stage is
 // this file's kernel too, else the 2-D resp. 3-D transform.
+// A transform that the x line kernels run instead (both in FP32, the forward
+// one in FP64) gets no plan: its handle stays 0.
 static bool make_plans(const x3d_ctx* c, hipfftHandle* r2c, hipfftHandle* c2r, hipfftType tr, hipfftType tc)
 {
   const int nx = c->nx, ny = c->ny, nz = c->nz, nxh = nx / 2 + 1;
+  if (c->xsplit) {
+    if (tc == HIPFFT_C2R) return true;
+    int n1[1] = {nx}, re1[1] = {nx}, ce1[1] = {nxh};
+    return hipfftPlanMany(c2r, 1, n1, ce1, 1, nxh, re1, 1, nx, tc, ny * nz) == HIPFFT_SUCCESS;
+  }
   int n2[2] = {ny, nx}, re2[2] = {ny, nx}, ce2[2] = {ny, nxh};
   const int rd = nx * ny, cd = nxh * ny;
   if (c->zsplit) {
@@ -1251,7 +1258,10 @@ static bool make_plans(const x3d_ctx* c, hipfftHandle* r2c, hipfftHandle* c2r, h
   } else {
     ok = hipfftPlan3d(c2r, nz, ny, nx, tc) == HIPFFT_SUCCESS;
   }
-  if (!ok) hipfftDestroy(*r2c);
+  if (!ok) {
+    hipfftDestroy(*r2c);
+    *r2c = 0;
+  }
   return ok;
 }
 
@@ -1326,23 +1336,25 @@ int poisson_setup(x3d_ctx* c)
     }
   }
   c->fft_ready = true;
-  if (hipfftSetStream(c->fft_r2c, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
-  if (hipfftSetStream(c->fft_c2r, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
+  return fft_streams(c, c->stream);
+}
+
+int fft_streams(x3d_ctx* c, hipStream_t s)
+{
+  const hipfftHandle plans[4] = {c->fft_ready ? c->fft_r2c : 0, c->fft_ready ? c->fft_c2r : 0,
+                                 c->fft32_ready ? c->fft_r2c32 : 0, c->fft32_ready ? c->fft_c2r32 : 0};
+  for (hipfftHandle p : plans)
+    if (p && hipfftSetStream(p, s) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
   return X3D_OK;
 }
 
 void poisson_release(x3d_ctx* c)
 {
-  if (c->fft_ready) {
-    hipfftDestroy(c->fft_r2c);
-    hipfftDestroy(c->fft_c2r);
-    c->fft_ready = false;
+  for (hipfftHandle* p : {&c->fft_r2c, &c->fft_c2r, &c->fft_r2c32, &c->fft_c2r32}) {
+    if (*p) hipfftDestroy(*p);
+    *p = 0;
   }
-  if (c->fft32_ready) {
-    hipfftDestroy(c->fft_r2c32);
-    hipfftDestroy(c->fft_c2r32);
-    c->fft32_ready = false;
-  }
+  c->fft_ready = c->fft32_ready = false;
   if (c->spec) (void)hipFree(c->spec);
   if (c->ktab) (void)hipFree(c->ktab);
   if (c->ztw) (void)hipFree(c->ztw);
@@ -1411,8 +1423,7 @@ int poisson_solve_f32(x3d_ctx* c, float* rhs)
 {
   const int rc = poisson_prepare_f32(c);
   if (rc) return rc;
-  if (hipfftSetStream(c->fft_r2c32, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
-  if (hipfftSetStream(c->fft_c2r32, c->stream) != HIPFFT_SUCCESS) return X3D_ERR_FFT;
+  if (const int rs = fft_streams(c, c->stream)) return rs;
   // the FP64 spectrum buffer holds the FP32 one
   float2* spec = reinterpret_cast<float2*>(c->spec);
   if (c->xsplit) {
