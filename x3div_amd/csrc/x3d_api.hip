@@ -169,7 +169,8 @@ static void np_direction_ops(x3d_ctx* c, int d, int n, int ncl1, int ncln)
 }
 
 // The non-periodic instances' tables padded to their direction's C*M points
-// with identity rows (f = s = 0, w = 1), in one device array.
+// with identity rows (f = s = 0, w = 1), in one device array; x: point k of
+// chunk c is entry k C + c (consecutive lanes hold consecutive chunks).
 static int np_upload(x3d_ctx* c)
 {
   std::vector<double> host;
@@ -181,11 +182,13 @@ static int np_upload(x3d_ctx* c)
     o.npoff = host.size();
     host.resize(host.size() + 3 * np, 0.0);
     double* f = host.data() + o.npoff;
+    const size_t C = (size_t)c->npplan[d].C, M = (size_t)c->npplan[d].M;
     for (size_t j = 0; j < np; ++j) {
       const bool real = j < (size_t)o.n;
-      f[j] = real ? o.f[j] : 0.0;
-      f[np + j] = real ? o.s[j] : 0.0;
-      f[2 * np + j] = real ? o.w[j] : 1.0;
+      const size_t q = d == 0 ? (j % M) * C + j / M : j;
+      f[q] = real ? o.f[j] : 0.0;
+      f[np + q] = real ? o.s[j] : 0.0;
+      f[2 * np + q] = real ? o.w[j] : 1.0;
     }
   }
   if (host.empty()) return X3D_OK;

@@ -2,6 +2,7 @@
 // tridiagonal solve and store, one pass over each line (one read of the
 // input window, one write).  Drop-ins for derx_00/dery_00/derz_00, the twelve
 // staggered routines and xthomas_0/ythomas_0/zthomas_0.
+#include <algorithm>
 #include <cmath>
 
 #include <cstdio>
@@ -123,16 +124,122 @@ __device__ __forceinline__ double np_rhs(const double* w, int q, int j, int n, c
   return -r.afn * w[q] - r.bfn * w[q - 1] - r.cfn * w[q - 2];
 }
 
+// LDS index of point e of a wavefront's run of x-lines: one word in 17 is left
+// out, so that chunks of 8 or 16 points do not start on the same banks.
+__device__ __forceinline__ int np_slot(int e) { return e + (e >> 4); }
+template <int M>
+constexpr int np_tile_words() { return 64 * M + 4 * M; }
+
+// Points of this wavefront's run of x-lines that belong to lines of the field,
+// and the byte offset of its first one.
+__device__ __forceinline__ int np_run(const Geom& geo, const LineThread& t, int n, uint32_t* base)
+{
+  const int first = t.line - t.lineLocal;
+  *base = (uint32_t)first * (uint32_t)n * 8u;
+  return max(0, min(t.LW, geo.nlines - first)) * n;
+}
+
+// This lane's chunk of the right-hand side (RHS), or of the field itself, from
+// its wavefront's run of x-lines.
+template <int M, bool RHS>
+__device__ __forceinline__ void np_chunk_x(const double* in, const NpRows& r, const Geom& geo, const LineThread& t,
+                                           double* tile, double (&v)[M])
+{
+  constexpr int H = RHS ? 2 : 0;
+  const int n = r.n, c = t.c, lane = threadIdx.x & 63, line0 = t.lineLocal * n;
+  double win[M + 2 * H];
+  // (a run has at most 64 M points: C M >= n)
+  uint32_t base;
+  const int run = np_run(geo, t, n, &base);
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    const int e = lane + 64 * k;
+    v[k] = 0.0;
+    if (e < run) v[k] = ld(in, base + (uint32_t)e * 8u);
+  }
+#pragma unroll
+  for (int k = 0; k < M; ++k) tile[np_slot(lane + 64 * k)] = v[k];
+  wave_lds_sync();
+#pragma unroll
+  for (int q = 0; q < M + 2 * H; ++q) {
+    int j = t.j0 - H + q;
+    j = j < 0 ? 0 : (j > n - 1 ? n - 1 : j);
+    win[q] = tile[np_slot(line0 + j)];
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    if constexpr (RHS) v[k] = r.afi * (win[k + 3] - win[k + 1]) + r.bfi * (win[k + 4] - win[k]);
+    else v[k] = win[k];
+  }
+  // boundary rows, each formed for every lane with uniform branches only and
+  // kept by the chunk that holds it (every x wavefront holds both ends), and
+  // zeros past the line's end
+  if constexpr (RHS) {
+    const double x0 = np_rhs(win, H, 0, n, r);
+    if constexpr (M > 1) {
+      const double x1 = np_rhs(win, 1 + H, 1, n, r);
+      v[0] = c == 0 ? x0 : v[0];
+      v[1] = c == 0 ? x1 : v[1];
+    } else {
+      const double x1 = np_rhs(win, H, 1, n, r);
+      v[0] = c == 0 ? x0 : (c == 1 ? x1 : v[0]);
+    }
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      if (k == (n - 2) % M) {
+        const double x = np_rhs(win, k + H, n - 2, n, r);
+        v[k] = t.j0 + k == n - 2 ? x : v[k];
+      }
+      if (k == (n - 1) % M) {
+        const double x = np_rhs(win, k + H, n - 1, n, r);
+        v[k] = t.j0 + k == n - 1 ? x : v[k];
+      }
+    }
+  }
+  if (t.C * M > n) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) v[k] = t.j0 + k < n ? v[k] : 0.0;
+  }
+}
+
+template <int M>
+__device__ __forceinline__ void np_store_x(double* out, const Geom& geo, const LineThread& t, int n, double* tile,
+                                           const double (&v)[M])
+{
+  const int lane = threadIdx.x & 63, line0 = t.lineLocal * n;
+  uint32_t base;
+  const int run = np_run(geo, t, n, &base);
+#pragma unroll
+  for (int k = 0; k < M; ++k)
+    if (t.j0 + k < n) tile[np_slot(line0 + t.j0 + k)] = v[k];
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    const int e = lane + 64 * k;
+    if (e < run) st(out, base + (uint32_t)e * 8u, tile[np_slot(e)]);
+  }
+}
+
 // One non-periodic first derivative along x, y or z (RHS), or the Thomas
 // sweeps alone: the right-hand side, then the reference's sweeps with the
 // instance's tables and no periodic correction (xthomas_12,
-// src/thomas.f90:61-84).  Lines have any length n: they are cut into C
-// chunks of M points with C M >= n, and the points past n are identity rows
-// of the padded tables (f = s = 0, w = 1) with a zero right-hand side, which
-// the sweeps carry through without touching the real points (f(n-1) = 0).
-// Every load is clamped into the line (the clamped values feed no real row)
-// and only real points are stored.  The Thomas form reads its own chunk
-// alone, so it may run in place.
+// src/thomas.f90:61-84), reassociated into chunked first-order recurrences as
+// in solve_table.  Lines have any length n: they are cut into C chunks of M
+// points with C M >= n, and the points past n are identity rows of the padded
+// tables (f = s = 0, w = 1) with a zero right-hand side, which the sweeps
+// carry through without touching the real points (f(n-1) = 0).  Every load is
+// clamped into the line (the clamped values feed no real row) and only real
+// points are stored.  The Thomas form reads its own chunk alone, so it may run
+// in place.
+// A wavefront's x-lines are one contiguous run of LW n points, read and
+// written lane by lane through an LDS tile, and their tables are stored chunk
+// point by chunk point: a lane's own chunk of field or tables lies M points
+// from its neighbour's, so that an access touched 64 cache lines.  513 x 257 x
+// 129, x: 97 -> 66 us; 128 x 256 x 512: 140 -> 54.
+// (y/z with LDS tables and persistent work-groups: 102 -> 82 us at 9-point
+// chunks, but 52 -> 93 at 16-point ones and slower on small grids; boundary
+// rows with uniform branches there: spills.)
 template <int M, bool LF, bool RHS>
 __global__ __launch_bounds__(LF ? 1024 : 256) void k_der_np(const double* in, double* out, OpDev<double> op, NpRows r,
                                                             Geom geo, Tiling tl)
@@ -140,34 +247,41 @@ __global__ __launch_bounds__(LF ? 1024 : 256) void k_der_np(const double* in, do
   constexpr int H = RHS ? 2 : 0;
   extern __shared__ unsigned char smem_raw[];
   double* lds = reinterpret_cast<double*>(smem_raw);
-  const LineThread t = line_thread<double>(geo, tl, M, blockIdx.x);
+  const LineThread t = line_thread<double>(geo, tl, M, tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x);
   const int n = r.n;
   double v[M];
-  {
-    double win[M + 2 * H];
+  if constexpr (!LF) {
+    double* const tile = lds + (threadIdx.x >> 6) * np_tile_words<M>();
+    np_chunk_x<M, RHS>(in, r, geo, t, tile, v);
+    solve_table<double, M, false, true>(v, t, op, lds, t.C * M, false);
+    np_store_x<M>(out, geo, t, n, tile, v);
+  } else {
+    {
+      double win[M + 2 * H];
 #pragma unroll
-    for (int q = 0; q < M + 2 * H; ++q) {
-      int j = t.j0 - H + q;
-      j = j < 0 ? 0 : (j > n - 1 ? n - 1 : j);
-      win[q] = ld(in, t.at(j));
-    }
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-      const int j = t.j0 + k;
-      double x = 0.0;
-      if constexpr (RHS) {
-        if (j < n) x = np_rhs(win, k + H, j, n, r);
-      } else {
-        if (j < n) x = win[k];
+      for (int q = 0; q < M + 2 * H; ++q) {
+        int j = t.j0 - H + q;
+        j = j < 0 ? 0 : (j > n - 1 ? n - 1 : j);
+        win[q] = ld(in, t.at(j));
       }
-      v[k] = x;
-    }
-  }
-  solve_table<double, M, LF>(v, t, op, lds, t.C * M, false);
-  if (t.active) {
 #pragma unroll
-    for (int k = 0; k < M; ++k)
-      if (t.j0 + k < n) st(out, t.at(t.j0 + k), v[k]);
+      for (int k = 0; k < M; ++k) {
+        const int j = t.j0 + k;
+        double x = 0.0;
+        if constexpr (RHS) {
+          if (j < n) x = np_rhs(win, k + H, j, n, r);
+        } else {
+          if (j < n) x = win[k];
+        }
+        v[k] = x;
+      }
+    }
+    solve_table<double, M, true>(v, t, op, lds, t.C * M, false);
+    if (t.active) {
+#pragma unroll
+      for (int k = 0; k < M; ++k)
+        if (t.j0 + k < n) st(out, t.at(t.j0 + k), v[k]);
+    }
   }
 }
 
@@ -539,15 +653,19 @@ NpRows np_rows(const x3d_ctx* c, int dir, int op)
 }
 
 // Chunking of a non-periodic line of any length n >= 8: C chunks (a power of
-// two up to 64) of M <= 16 points with C M >= n and the least padding; y/z
-// take up to 4 chunk groups per wavefront and C / 4 wavefronts per line set.
+// two up to 64) of M <= 16 points with C M >= n and the least padding; x
+// counts chunks of more than 10 points a third longer, as their kernels hold
+// fewer wavefronts; y/z take up to 4 chunk groups per wavefront and C / 4
+// wavefronts per line set.
 int np_plan(int n, bool line_fast, LinePlan* P)
 {
   if (n < 8) return X3D_ERR_SIZE;
-  int C = 0, M = 0, pad = 1 << 30;
+  int C = 0, M = 0, least = 1 << 30;
   for (int c = 1; c <= 64; c <<= 1)
-    for (int m = 1; m <= 16; ++m)
-      if (c * m >= n && c * m - n < pad) { C = c; M = m; pad = c * m - n; }
+    for (int m = 1; m <= 16; ++m) {
+      const int cost = c * m * (m > 10 && !line_fast ? 4 : 3);
+      if (c * m >= n && cost < least) { C = c; M = m; least = cost; }
+    }
   if (!C) return X3D_ERR_UNSUPPORTED;
   LinePlan p;
   p.n = n; p.M = M; p.C = C; p.line_fast = line_fast;
@@ -578,8 +696,11 @@ int launch_line_np(x3d_ctx* c, int dir, int op, const double* in, double* out, b
   dim3 grid, block;
   size_t smem;
   launch_dims_plan(c, dir, P, &geo, &tl, &grid, &block, &smem, sizeof(double));
-  tl.xcd = 0;
-  if (!P.line_fast) smem = 0;  // x-lines: no staging tile, and the sweeps stay in the wavefront
+  // strided blocks whose rows do not start on cache lines share them with their
+  // neighbours: regrouped per XCD, so that one L2 holds them (513 x 257 x 129:
+  // y 104 -> 94 us, z 118 -> 95)
+  tl.xcd = dir && c->nx % 16 ? c->xcd_remap : 0;
+  if (!P.line_fast) smem = sizeof(double) * (size_t)(P.Wc * P.Wl) * (size_t)(68 * P.M);  // x: a tile per wavefront
   const size_t np = (size_t)P.C * P.M;
   const double* tb = c->nptab + c->op[op].npoff;
   const OpDev<double> od{tb, tb + np, tb + 2 * np, nullptr, c->op[op].alfa};

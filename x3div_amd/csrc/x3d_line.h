@@ -752,11 +752,14 @@ __device__ __forceinline__ void solve_circ(T (&v)[M], const LineThread& t, const
 }
 
 // ---- table solver (the reference's sweeps with the operator's vectors) -------
-template <typename T, int M, bool LF>
+// TR: the vectors f, s, w are stored chunk point by chunk point, entry k of
+// chunk c at k C + c, so that the lanes of a wavefront read neighbouring words.
+template <typename T, int M, bool LF, bool TR = false>
 __device__ __forceinline__ void solve_table(T (&v)[M], const LineThread& t, const OpDev<T>& op, T* lds,
                                             int n, bool fix)
 {
   const int G = t.G, g = t.g, Wc = LF ? t.Wc : 1, LPW = t.LPW, ls = t.ls, j0 = t.j0;
+  auto at = [&](int k) { return TR ? k * t.C + t.c : j0 + k; };
   T* sA = lds;
   T* sB = sA + Wc * LPW;
   T* rA = sB + Wc * LPW;
@@ -770,7 +773,7 @@ __device__ __forceinline__ void solve_table(T (&v)[M], const LineThread& t, cons
     T prev = T(0);
 #pragma unroll
     for (int k = 0; k < M; ++k) {
-      const T s = op.s[j0 + k];
+      const T s = op.s[at(k)];
       v[k] = v[k] - prev * s;
       prev = v[k];
       A = A * (-s);
@@ -801,7 +804,7 @@ __device__ __forceinline__ void solve_table(T (&v)[M], const LineThread& t, cons
     T P = T(1);
 #pragma unroll
     for (int k = 0; k < M; ++k) {
-      P = P * (-op.s[j0 + k]);
+      P = P * (-op.s[at(k)]);
       v[k] = v[k] + P * carry;
     }
   }
@@ -812,7 +815,7 @@ __device__ __forceinline__ void solve_table(T (&v)[M], const LineThread& t, cons
     T nxt = T(0);
 #pragma unroll
     for (int k = M - 1; k >= 0; --k) {
-      const T f = op.f[j0 + k], w = op.w[j0 + k];
+      const T f = op.f[at(k)], w = op.w[at(k)];
       v[k] = (v[k] - f * nxt) * w;
       nxt = v[k];
       A = A * (-(f * w));
@@ -842,7 +845,7 @@ __device__ __forceinline__ void solve_table(T (&v)[M], const LineThread& t, cons
     T Q = T(1);
 #pragma unroll
     for (int k = M - 1; k >= 0; --k) {
-      const T f = op.f[j0 + k], w = op.w[j0 + k];
+      const T f = op.f[at(k)], w = op.w[at(k)];
       Q = Q * (-(f * w));
       v[k] = v[k] + Q * carry;
     }
