@@ -51,6 +51,20 @@ struct DivXArgs {
   Circ<T> cci;
 };
 
+// Right-hand side of D(u_d u_c).  The products are rounded once each: left to
+// the compiler, which of them fuse into the differences depended on the kernel
+// around it, and the step and the pieces it stands for differed in last bits.
+template <typename T, int M>
+__device__ __forceinline__ void product_rhs(const T (&wd)[M + 4], const T (&wc)[M + 4], const Coef<T>& cf, T (&v)[M])
+{
+#pragma clang fp contract(off)
+  T p[M + 4];
+#pragma unroll
+  for (int q = 0; q < M + 4; ++q) p[q] = wd[q] * wc[q];
+#pragma unroll
+  for (int k = 0; k < M; ++k) v[k] = fma(cf.b, p[k + 4] - p[k], cf.a * (p[k + 3] - p[k + 1]));
+}
+
 // DX (last x pass of a step): each updated u_c is in the staging tile when it
 // has been stored, so the x operators of the divergence, whose lines are the
 // same, take it from there: the pass writes their three results (15 fields
@@ -143,12 +157,7 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
         }
       }
       rhs_chunk<K_D, T, M, H>(wc, cf, v2);
-#pragma unroll
-      for (int k = 0; k < M; ++k) {
-        const int q = k + H;
-        v1[k] = cf.a * (wd[q + 1] * wc[q + 1] - wd[q - 1] * wc[q - 1]) +
-                cf.b * (wd[q + 2] * wc[q + 2] - wd[q - 2] * wc[q - 2]);
-      }
+      product_rhs<T, M>(wd, wc, cf, v1);
     }
     // y: the epilogue's strided loads (du_c of the z pass) are issued here and
     // complete during the two line solves, whose barriers wait on LDS only.

@@ -47,23 +47,27 @@ struct Coef { T a, b, c, d; };
 // DD   derxx        (declared only, src/x3d_derive.f90:54-59): sixth-order
 //                   compact second derivative, a (u+1 - 2u + u-1) + b (u+2 - 2u + u-2)
 // (the wrapped boundary rows are the same formulas with indices mod n)
+// The fused multiply-adds are written out: which of two products the compiler
+// fuses into their sum depends on the code around it, and kernels that compute
+// the same values (a fused pass and the passes it stands for) would differ in
+// their last bits.
 template <int KIND, typename T>
 __device__ __forceinline__ T rhs_at(const T* win, int q, const Coef<T>& k)
 {
   if constexpr (KIND == K_D)
-    return k.a * (win[q + 1] - win[q - 1]) + k.b * (win[q + 2] - win[q - 2]);
+    return fma(k.a, win[q + 1] - win[q - 1], k.b * (win[q + 2] - win[q - 2]));
   else if constexpr (KIND == K_DVP)
-    return k.a * (win[q + 1] - win[q]) + k.b * (win[q + 2] - win[q - 1]);
+    return fma(k.a, win[q + 1] - win[q], k.b * (win[q + 2] - win[q - 1]));
   else if constexpr (KIND == K_DPV)
-    return k.a * (win[q] - win[q - 1]) + k.b * (win[q + 1] - win[q - 2]);
+    return fma(k.a, win[q] - win[q - 1], k.b * (win[q + 1] - win[q - 2]));
   else if constexpr (KIND == K_IVP)
-    return k.a * (win[q + 1] + win[q]) + k.b * (win[q + 2] + win[q - 1]) +
-           k.c * (win[q + 3] + win[q - 2]) + k.d * (win[q + 4] + win[q - 3]);
+    return fma(k.d, win[q + 4] + win[q - 3], fma(k.c, win[q + 3] + win[q - 2],
+               fma(k.a, win[q + 1] + win[q], k.b * (win[q + 2] + win[q - 1]))));
   else if constexpr (KIND == K_IPV)
-    return k.a * (win[q] + win[q - 1]) + k.b * (win[q + 1] + win[q - 2]) +
-           k.c * (win[q + 2] + win[q - 3]) + k.d * (win[q + 3] + win[q - 4]);
+    return fma(k.d, win[q + 3] + win[q - 4], fma(k.c, win[q + 2] + win[q - 3],
+               fma(k.a, win[q] + win[q - 1], k.b * (win[q + 1] + win[q - 2]))));
   else if constexpr (KIND == K_DD)
-    return k.a * ((win[q + 1] + win[q - 1]) - (T)2 * win[q]) + k.b * ((win[q + 2] + win[q - 2]) - (T)2 * win[q]);
+    return fma(k.a, fma((T)-2, win[q], win[q + 1] + win[q - 1]), k.b * fma((T)-2, win[q], win[q + 2] + win[q - 2]));
   else
     return win[q];
 }
