@@ -3,8 +3,8 @@
 // (products, combinations, Euler update, velocity correction) folded into the
 // prologue/epilogue.  At one rank the pencils are one array, so the step is
 //   transeq   Z -> Y -> X(+combine, Euler)        src/transeq.f90:44-355
-//             (FP32 single grids: X -> Y -> Z(+combine, Euler))
 //   divergence X -> Y -> Z                         src/navier.f90:98-236
+//             (a step's X rides in transeq's X, except in BFP32)
 //   Poisson                                        src/poisson.f90:276-419
 //   gradp     Z -> Y -> X(+cor_vel)                src/navier.f90:249-359, 64-91
 // Each pass reads its input fields once and writes its outputs once; all
@@ -70,10 +70,13 @@ __device__ __forceinline__ void product_rhs(const T (&wd)[M + 4], const T (&wc)[
 // same, take it from there: the pass writes their three results (15 fields
 // with the rest) and the divergence's own x pass, which would read u again (6
 // fields), falls away.  What bounds it is HBM, 15 fields at the copy rate.
-template <typename S, int M, int DIR, bool DX = false>
+// PART >= 0 (y and z passes): the component PART alone, for split launches.
+template <typename S, int M, int DIR, bool DX = false, int PART = -1>
 __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ A, int blk,
                                              const DivXArgs<S>* __restrict__ X = nullptr)
 {
+  static_assert(PART < 0 || DIR != 0, "the x pass updates u in place: one work-group takes all components");
+  constexpr int C0 = PART < 0 ? 0 : PART, C1 = PART < 0 ? 3 : PART + 1;
   using T = typename Store<S>::T;
   S* const ux = A.ux; S* const uy = A.uy; S* const uz = A.uz;
   S* const dux = A.dux; S* const duy = A.duy; S* const duz = A.duz;
@@ -110,10 +113,10 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
   // BFP32 fields) with 16-point chunks only, whose 512-thread work-groups
   // hold 2 waves per SIMD with or without the window's registers (shorter
   // chunks would lose occupancy).
-  constexpr bool PREW = DIR == 2 && sizeof(T) == 8 && M >= 16;
+  constexpr bool PREW = DIR == 2 && sizeof(T) == 8 && M >= 16 && PART < 0;
   RawT<S> pw[PREW ? NW : 1];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
+  for (int c = C0; c < C1; ++c) {
     // components one after another: no loads hoisted across them
     __builtin_amdgcn_sched_barrier(0);
     // pointers straight from the kernel arguments (c is a constant here)
@@ -134,7 +137,7 @@ __device__ __forceinline__ void transeq_body(const TranseqArgs<S>& __restrict__ 
           x_load_window<S, M, H, H>(Uc, xb, t, wc);
         }
       } else {
-        if (c == 0) {
+        if (c == C0) {
           load_window<S, M, H, H, true>(Ud, t, n, wd);
 #pragma unroll
           for (int q = 0; q < NW; ++q) keep[q * nth + tid] = wd[q];
@@ -276,9 +279,11 @@ struct PassArgs {
   const T* sy;  // y-stretching: ppyi(j) for Dvp (divergence), ppy(j) for Dpv (gradp), or nullptr
 };
 
-template <typename S, int M, int DIR>
+// PART >= 0 (y): output PART alone.
+template <typename S, int M, int DIR, int PART = -1>
 __device__ __forceinline__ void div_body(const PassArgs<S>& __restrict__ A, int blk)
 {
+  static_assert(PART < 0 || DIR == 1, "the y pass has two independent outputs");
   using T = typename Store<S>::T;
   const S* const a = A.a; const S* const b = A.b; const S* const c = A.c;
   S* const o1 = A.o1; S* const o2 = A.o2; S* const o3 = A.o3;
@@ -315,33 +320,38 @@ __device__ __forceinline__ void div_body(const PassArgs<S>& __restrict__ A, int 
     solve_circ<T, M, false>(v, t, cci, lds);
     x_store<S, M>(o3, xb, v);
   } else if constexpr (DIR == 1) {
-    T v[M], s[M];
-    {
-      T w[M + 3];
-      load_window<S, M, 1, 2, DIR != 0>(b, t, n, w);
-      rhs_chunk<K_DVP, T, M, 1>(w, cfd, v);
-    }
-    solve_circ<T, M, DIR != 0>(v, t, ccd, lds);
-    if (A.sy) {
+    T v[M];
+    if constexpr (PART != 1) {
+      T s[M];
+      {
+        T w[M + 3];
+        load_window<S, M, 1, 2, DIR != 0>(b, t, n, w);
+        rhs_chunk<K_DVP, T, M, 1>(w, cfd, v);
+      }
+      solve_circ<T, M, DIR != 0>(v, t, ccd, lds);
+      if (A.sy) {
 #pragma unroll
-      for (int k = 0; k < M; ++k) v[k] = v[k] * A.sy[t.j0 + k];
-    }
-    {
-      T w[M + 7];
-      load_window<S, M, 3, 4, DIR != 0>(a, t, n, w);
-      rhs_chunk<K_IVP, T, M, 3>(w, cfi, s);
-    }
-    solve_circ<T, M, DIR != 0>(s, t, cci, lds);
+        for (int k = 0; k < M; ++k) v[k] = v[k] * A.sy[t.j0 + k];
+      }
+      {
+        T w[M + 7];
+        load_window<S, M, 3, 4, DIR != 0>(a, t, n, w);
+        rhs_chunk<K_IVP, T, M, 3>(w, cfi, s);
+      }
+      solve_circ<T, M, DIR != 0>(s, t, cci, lds);
 #pragma unroll
-    for (int k = 0; k < M; ++k) v[k] = v[k] + s[k];
-    store_chunk<S, M>(o1, t, v);
-    {
-      T w[M + 7];
-      load_window<S, M, 3, 4, DIR != 0>(c, t, n, w);
-      rhs_chunk<K_IVP, T, M, 3>(w, cfi, v);
+      for (int k = 0; k < M; ++k) v[k] = v[k] + s[k];
+      store_chunk<S, M>(o1, t, v);
     }
-    solve_circ<T, M, DIR != 0>(v, t, cci, lds);
-    store_chunk<S, M>(o2, t, v);
+    if constexpr (PART != 0) {
+      {
+        T w[M + 7];
+        load_window<S, M, 3, 4, DIR != 0>(c, t, n, w);
+        rhs_chunk<K_IVP, T, M, 3>(w, cfi, v);
+      }
+      solve_circ<T, M, DIR != 0>(v, t, cci, lds);
+      store_chunk<S, M>(o2, t, v);
+    }
   } else {
     T v[M], s[M];
     {
@@ -373,7 +383,8 @@ __device__ __forceinline__ void div_body(const PassArgs<S>& __restrict__ A, int 
 // Y: o1 = Ipv(a), o2 = Dpv(a), o3 = Ipv(b)          a, b = ppi3, pgz3
 // X: o1 = Dpv(a), o2 = Ipv(b), o3 = Ipv(c)          a, b, c = ppi2, pgy2, pgzi2
 //    if corr: u_k = u_k - o_k (src/navier.f90:84-86)
-template <typename S, int M, int DIR>
+// PART >= 0: output PART alone.
+template <typename S, int M, int DIR, int PART = -1>
 __device__ __forceinline__ void grad_body(const PassArgs<S>& __restrict__ A, int blk)
 {
   using T = typename Store<S>::T;
@@ -391,22 +402,26 @@ __device__ __forceinline__ void grad_body(const PassArgs<S>& __restrict__ A, int
   const int n = geo.n;
   if constexpr (DIR == 2 || DIR == 1) {
     T v[M];
-    {
+    if constexpr (PART != 2) {
       T w[M + 7];
       load_window<S, M, 4, 3, DIR != 0>(a, t, n, w);
-      rhs_chunk<K_IPV, T, M, 4>(w, cfi, v);
       T s[M];
-      rhs_chunk<K_DPV, T, M, 4>(w, cfd, s);
-      solve_circ<T, M, DIR != 0>(v, t, cci, lds);
-      store_chunk<S, M>(o1, t, v);
-      solve_circ<T, M, DIR != 0>(s, t, ccd, lds);
-      if (DIR == 1 && A.sy) {
-#pragma unroll
-        for (int k = 0; k < M; ++k) s[k] = s[k] * A.sy[t.j0 + k];
+      if constexpr (PART != 1) rhs_chunk<K_IPV, T, M, 4>(w, cfi, v);
+      if constexpr (PART != 0) rhs_chunk<K_DPV, T, M, 4>(w, cfd, s);
+      if constexpr (PART != 1) {
+        solve_circ<T, M, DIR != 0>(v, t, cci, lds);
+        store_chunk<S, M>(o1, t, v);
       }
-      store_chunk<S, M>(o2, t, s);
+      if constexpr (PART != 0) {
+        solve_circ<T, M, DIR != 0>(s, t, ccd, lds);
+        if (DIR == 1 && A.sy) {
+#pragma unroll
+          for (int k = 0; k < M; ++k) s[k] = s[k] * A.sy[t.j0 + k];
+        }
+        store_chunk<S, M>(o2, t, s);
+      }
     }
-    if constexpr (DIR == 1) {
+    if constexpr (DIR == 1 && (PART < 0 || PART == 2)) {
       T w[M + 7];
       load_window<S, M, 4, 3, DIR != 0>(b, t, n, w);
       rhs_chunk<K_IPV, T, M, 4>(w, cfi, v);
@@ -416,7 +431,7 @@ __device__ __forceinline__ void grad_body(const PassArgs<S>& __restrict__ A, int
   } else {
     const XBlock<S, M> xb = x_block<S, M>(geo, t, lds);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int q = PART < 0 ? 0 : PART; q < (PART < 0 ? 3 : PART + 1); ++q) {
       const S* const inq = q == 0 ? a : (q == 1 ? b : c);
       S* const outq = q == 0 ? o1 : (q == 1 ? o2 : o3);
       S* const Uq = q == 0 ? ux : (q == 1 ? uy : uz);
@@ -468,6 +483,31 @@ template <typename S, int M, int DIR>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DIR == 1 ? 4 : 1))) void k_div(PassArgs<S> A) { div_body<S, M, DIR>(A, A.tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x); }
 template <typename S, int M, int DIR>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DIR == 1 ? 4 : 1))) void k_grad(PassArgs<S> A) { grad_body<S, M, DIR>(A, A.tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x); }
+
+// Split launches, for grids whose passes leave SIMDs without a wavefront:
+// blockIdx.y is the component (transeq y, z), the output (divergence y: 2,
+// gradient: 2 along z, else 3), each with its own work-groups instead of one
+// after another.  The inputs they share are read again, from cache.
+template <typename S, int M, int DIR>
+__global__ __launch_bounds__(512) void k_transeq_split(TranseqArgs<S> A)
+{
+  if (blockIdx.y == 0) transeq_body<S, M, DIR, false, 0>(A, blockIdx.x);
+  else if (blockIdx.y == 1) transeq_body<S, M, DIR, false, 1>(A, blockIdx.x);
+  else transeq_body<S, M, DIR, false, 2>(A, blockIdx.x);
+}
+template <typename S, int M>
+__global__ __launch_bounds__(512) void k_div_y_split(PassArgs<S> A)
+{
+  if (blockIdx.y == 0) div_body<S, M, 1, 0>(A, blockIdx.x);
+  else div_body<S, M, 1, 1>(A, blockIdx.x);
+}
+template <typename S, int M, int DIR>
+__global__ __launch_bounds__(512) void k_grad_split(PassArgs<S> A)
+{
+  if (blockIdx.y == 0) grad_body<S, M, DIR, 0>(A, blockIdx.x);
+  else if (DIR == 2 || blockIdx.y == 1) grad_body<S, M, DIR, 1>(A, blockIdx.x);
+  else if constexpr (DIR != 2) grad_body<S, M, DIR, 2>(A, blockIdx.x);
+}
 
 template <typename T, int M, int DIR>
 __global__ __launch_bounds__(512) void k_transeq_batch(const TranseqArgs<T>* __restrict__ list,
@@ -624,6 +664,24 @@ static bool storage_ok(const x3d_ctx* c, int dir)
   return c->nx % 16 == 0 && (!P.line_fast || P.bfp);
 }
 
+// Whether a pass over a small grid runs with its outputs in blockIdx.y, one
+// work-group for each, instead of one after another in a work-group: the chain
+// of six line solves (transeq), three (divergence y, gradp x and y) or two
+// (gradp z) is cut to two or one, at the price of loading u_d (transeq) or the
+// input (gradp) again, which a small grid's caches give.  64^3 step: FP64 119
+// -> 97 us, FP32 101 -> 79.  It pays while the whole pass leaves SIMDs (4 per
+// compute unit) with one wavefront or none: FP64 up to 5 wavefronts per compute
+// unit (96^3 170 -> 161 us; at 8, 128^3 278 -> 285), FP32, whose wavefronts
+// need fewer registers, up to 7 (64 x 128 x 192 167 -> 162; at 8, 160^3 327 ->
+// 333).  Same arithmetic per output, so the results are bit for bit the same.
+// BFP32 fields keep one launch shape.
+template <typename S>
+static bool split_pass(const x3d_ctx* c, const DirSet<S>& s)
+{
+  const int waves_per_cu = sizeof(typename Store<S>::T) == 8 ? 5 : 7;
+  return !is_bfp<S> && (long long)s.grid.x * (s.block.x / 64) <= waves_per_cu * (long long)c->ncu;
+}
+
 template <int DIR, typename S>
 static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz, S* tx, S* ty, S* tz, double gdt,
                         int euler)
@@ -634,6 +692,16 @@ static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz,
   const TranseqArgs<S> A{ux,   uy,   uz,   dux,  duy,      duz,   tx,
                          ty,   tz,   s.cf_d, s.cc_d, s.geo, s.tl, (T)gdt,
                          euler, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
+  if constexpr (DIR != 0 && !is_bfp<S>) {
+    if (split_pass<S>(c, s)) {
+      X3D_MSWITCH_T(S, s.M, {
+        allow_lds((const void*)k_transeq_split<S, MM, DIR>, s.smem_tq);
+        hipLaunchKernelGGL((k_transeq_split<S, MM, DIR>), dim3(s.grid.x, 3), s.block, s.smem_tq, c->stream, A);
+      });
+      X3D_CHECK_HIP(hipGetLastError());
+      return X3D_OK;
+    }
+  }
   X3D_MSWITCH_T(S, s.M, {
     allow_lds((const void*)k_transeq<S, MM, DIR>, s.smem_tq);
     hipLaunchKernelGGL((k_transeq<S, MM, DIR>), s.grid, s.block, s.smem_tq, c->stream, A);
@@ -674,6 +742,13 @@ static int div_pass(x3d_ctx* c, const S* a, const S* b, const S* cc, S* o1, S* o
   const DirSet<S> s = dirset<S>(c, DIR);
   const PassArgs<S> A{a, b, cc, o1, o2, o3, nullptr, nullptr, nullptr, s.cf_dvp, s.cc_s, s.cf_ivp, s.cc_i,
                       s.geo, s.tl, 0, DIR == 1 ? stretch_vec<T>(c, 1) : nullptr};
+  if constexpr (DIR == 1 && !is_bfp<S>) {
+    if (split_pass<S>(c, s)) {
+      X3D_MSWITCH_T(S, s.M, hipLaunchKernelGGL((k_div_y_split<S, MM>), dim3(s.grid.x, 2), s.block, s.smem, c->stream, A));
+      X3D_CHECK_HIP(hipGetLastError());
+      return X3D_OK;
+    }
+  }
   X3D_MSWITCH_T(S, s.M, hipLaunchKernelGGL((k_div<S, MM, DIR>), s.grid, s.block, s.smem, c->stream, A));
   X3D_CHECK_HIP(hipGetLastError());
   return X3D_OK;
@@ -688,6 +763,16 @@ static int grad_pass(x3d_ctx* c, const S* a, const S* b, const S* cc, S* o1, S* 
   const DirSet<S> s = dirset<S>(c, DIR);
   const PassArgs<S> A{a,    b,    cc,       o1,     o2,       o3,     ux,    uy,   uz,
                       s.cf_dpv, s.cc_s, s.cf_ipv, s.cc_i, s.geo, s.tl, corr, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
+  if constexpr (!is_bfp<S>) {
+    // (x: outputs that a caller gave as one buffer are written in order)
+    if (split_pass<S>(c, s) && (DIR != 0 || (o1 != o2 && o1 != o3 && o2 != o3 && ux != o2 && ux != o3 && uy != o1 &&
+                                             uy != o3 && uz != o1 && uz != o2))) {
+      X3D_MSWITCH_T(S, s.M, hipLaunchKernelGGL((k_grad_split<S, MM, DIR>), dim3(s.grid.x, DIR == 2 ? 2 : 3), s.block,
+                                               s.smem, c->stream, A));
+      X3D_CHECK_HIP(hipGetLastError());
+      return X3D_OK;
+    }
+  }
   X3D_MSWITCH_T(S, s.M, hipLaunchKernelGGL((k_grad<S, MM, DIR>), s.grid, s.block, s.smem, c->stream, A));
   X3D_CHECK_HIP(hipGetLastError());
   return X3D_OK;
