@@ -246,14 +246,15 @@ int x3d_step(x3d_ctx *ctx, double gdt, double *ux, double *uy, double *uz,
 
 /* Per-pass timing of one step, the role of the reference's NVTX ranges
  * around each call of the step loop (src/xcompact3d.f90:79-93).  Runs
- * x3d_step with a HIP event after each of its X3D_NPASS passes on the
- * context's stream, waits for it, and writes each pass's milliseconds to
- * pass_ms[X3D_NPASS].  Pass i is named by x3d_pass_name(i); its algorithmic
- * HBM bytes per grid point (every field it reads or writes touched once) are
- * x3d_pass_bytes_per_point(i), in FP64.  The transeq passes run z, y, x: z
- * reads u and writes its part (6 fields), x adds the sum and the Euler update
- * (12 fields).  The FP32 form's single grids run them x, y, z: there
- * transeq_x moves 6 fields and transeq_z 12 (at 4 B each). */
+ * x3d_step's operations, with the same results, as X3D_NPASS passes with a HIP
+ * event after each on the context's stream, waits for them, and writes each
+ * pass's milliseconds to pass_ms[X3D_NPASS].  (x3d_step itself applies the
+ * divergence's x operators in the transeq x pass, in FP64 and FP32, and so
+ * moves 3 fields less than the ten passes together.)  Pass i is named by
+ * x3d_pass_name(i); its algorithmic HBM bytes per grid point (every field it
+ * reads or writes touched once) are x3d_pass_bytes_per_point(i), in FP64.  The
+ * transeq passes run z, y, x: z reads u and writes its part (6 fields), x adds
+ * the sum and the Euler update (12 fields). */
 #define X3D_NPASS 10
 int x3d_step_timed(x3d_ctx *ctx, double gdt, double *ux, double *uy, double *uz,
                    double *dux, double *duy, double *duz, double *pp3,
@@ -282,8 +283,9 @@ int x3d_poisson_f32(x3d_ctx *ctx, float *rhs);
  * FP64 from the reference's own periodic solve), applied to every line as a
  * GEMM on v_mfma_f32_32x32x16_f16 in three split-precision terms
  * (C_hi u_hi + C_hi u_lo + C_lo u_hi, fp16 halves after exact power-of-two
- * scaling, FP32 accumulation); a few 1e-6 relative to the FP64 operator.  Needs the line length a
- * multiple of 128 (at most 1024) and the line count a multiple of 32;
+ * scaling, FP32 accumulation), over the diagonals of C that are not zero in
+ * both halves; a few 1e-6 relative to the FP64 operator.  Needs the line
+ * length a multiple of 128 (at most 1024) and the line count a multiple of 32;
  * out != in. */
 int x3d_apply_circ_mfma(x3d_ctx *ctx, int op, float *out, const float *in);
 int x3d_step_f32(x3d_ctx *ctx, double gdt, float *ux, float *uy, float *uz,
