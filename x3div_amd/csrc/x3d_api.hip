@@ -322,15 +322,24 @@ template <bool SUB>
 static int update3(x3d_ctx* c, double* const (&o)[3], const double* const (&a)[3], double g)
 {
   const long long N = (long long)c->nx * c->ny * c->nz;
-  bool pair = true;
-  for (int k = 0; k < 3; ++k) pair = pair && !((reinterpret_cast<uintptr_t>(o[k]) | reinterpret_cast<uintptr_t>(a[k])) & 15);
+  bool pair = true, apart = true;
+  for (int k = 0; k < 3; ++k) {
+    pair = pair && !((reinterpret_cast<uintptr_t>(o[k]) | reinterpret_cast<uintptr_t>(a[k])) & 15);
+    for (int l = 0; l < 3; ++l)
+      if (l != k && (overlap(o[k], o[l], (size_t)N * 8) || overlap(o[k], a[l], (size_t)N * 8))) apart = false;
+  }
   const long long per = pair ? 512 : 256;
-  const dim3 grid((unsigned)std::min<long long>((N + per - 1) / per, 16384), 3);
-  if (pair)
-    hipLaunchKernelGGL((k_update3<SUB, true>), grid, dim3(256), 0, c->stream, o[0], o[1], o[2], a[0], a[1], a[2], g, N);
-  else
-    hipLaunchKernelGGL((k_update3<SUB, false>), grid, dim3(256), 0, c->stream, o[0], o[1], o[2], a[0], a[1], a[2], g, N);
-  X3D_CHECK_HIP(hipGetLastError());
+  // a component that updates another's operand (one buffer given for two of
+  // them): the components in order, one launch each
+  const dim3 grid((unsigned)std::min<long long>((N + per - 1) / per, 16384), apart ? 3 : 1);
+  for (int k = 0; k < (apart ? 1 : 3); ++k) {
+    const int k1 = apart ? 1 : k, k2 = apart ? 2 : k;
+    if (pair)
+      hipLaunchKernelGGL((k_update3<SUB, true>), grid, dim3(256), 0, c->stream, o[k], o[k1], o[k2], a[k], a[k1], a[k2], g, N);
+    else
+      hipLaunchKernelGGL((k_update3<SUB, false>), grid, dim3(256), 0, c->stream, o[k], o[k1], o[k2], a[k], a[k1], a[k2], g, N);
+    X3D_CHECK_HIP(hipGetLastError());
+  }
   return X3D_OK;
 }
 

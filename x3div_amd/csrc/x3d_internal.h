@@ -296,6 +296,13 @@ int poisson_batch_run(x3d_batch* b, int ns);
 
 int ensure_work(x3d_ctx* c);
 
+// Whether two arrays of `bytes` bytes each share memory.
+inline bool overlap(const void* a, const void* b, size_t bytes)
+{
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return (x < y ? y - x : x - y) < bytes;
+}
+
 // Record the end of step pass i (1-based) when x3d_step_timed is running.
 inline int mark_pass(x3d_ctx* c, int i)
 {
