@@ -682,9 +682,26 @@ static bool split_pass(const x3d_ctx* c, const DirSet<S>& s)
   return !is_bfp<S> && (long long)s.grid.x * (s.block.x / 64) <= waves_per_cu * (long long)c->ncu;
 }
 
+// Whether none of the outputs shares memory with another one or with an input.
+// Otherwise what a buffer holds in the end depends on the order in which the
+// outputs are written: such a call is not split, its outputs are written one
+// after another, the last one staying.
+template <typename S>
+static bool outputs_apart(const x3d_ctx* c, std::initializer_list<const S*> out, std::initializer_list<const S*> in)
+{
+  const size_t bytes = (size_t)c->nx * c->ny * c->nz * sizeof(S);
+  for (const S* const* o = out.begin(); o != out.end(); ++o) {
+    for (const S* const* q = o + 1; q != out.end(); ++q)
+      if (overlap(*o, *q, bytes)) return false;
+    for (const S* i : in)
+      if (overlap(*o, i, bytes)) return false;
+  }
+  return true;
+}
+
 template <int DIR, typename S>
 static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz, S* tx, S* ty, S* tz, double gdt,
-                        int euler)
+                        int euler, [[maybe_unused]] bool apart)
 {
   using T = typename Store<S>::T;
   if (!storage_ok<S>(c, DIR)) return X3D_ERR_UNSUPPORTED;
@@ -693,7 +710,7 @@ static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz,
                          ty,   tz,   s.cf_d, s.cc_d, s.geo, s.tl, (T)gdt,
                          euler, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
   if constexpr (DIR != 0 && !is_bfp<S>) {
-    if (split_pass<S>(c, s)) {
+    if (apart && split_pass<S>(c, s)) {
       X3D_MSWITCH_T(S, s.M, {
         allow_lds((const void*)k_transeq_split<S, MM, DIR>, s.smem_tq);
         hipLaunchKernelGGL((k_transeq_split<S, MM, DIR>), dim3(s.grid.x, 3), s.block, s.smem_tq, c->stream, A);
@@ -798,11 +815,12 @@ int fused_momentum(x3d_ctx* c, double gdt, int euler, T* ux, T* uy, T* uz, T* du
   if (sizeof(T) == 8 && !c->f64_lines) return X3D_ERR_UNSUPPORTED;
   X3D_TRY(ensure_work(c));
   T *tx = wk<T>(c, 5), *ty = wk<T>(c, 6), *tz = wk<T>(c, 7);
-  X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+  const bool apart = outputs_apart<T>(c, {dux, duy, duz}, {ux, uy, uz});
+  X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0, apart)));
   X3D_TRY(mark_pass(c, 1));
-  X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+  X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0, apart)));
   X3D_TRY(mark_pass(c, 2));
-  X3D_TRY((transeq_pass<0, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, euler)));
+  X3D_TRY((transeq_pass<0, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, euler, apart)));
   X3D_TRY(mark_pass(c, 3));
   return X3D_OK;
 }
@@ -847,8 +865,9 @@ int fused_momentum_divergence(x3d_ctx* c, double gdt, T* ux, T* uy, T* uz, T* du
     if (sizeof(T) == 8 && !c->f64_lines) return X3D_ERR_UNSUPPORTED;
     X3D_TRY(ensure_work(c));
     T *tx = wk<T>(c, 5), *ty = wk<T>(c, 6), *tz = wk<T>(c, 7);
-    X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
-    X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0)));
+    const bool apart = outputs_apart<T>(c, {dux, duy, duz}, {ux, uy, uz});
+    X3D_TRY((transeq_pass<2, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0, apart)));
+    X3D_TRY((transeq_pass<1, T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, 0, apart)));
     X3D_TRY((transeq_div_x_pass<T>(c, ux, uy, uz, dux, duy, duz, tx, ty, tz, gdt, wk<T>(c, 0), wk<T>(c, 1),
                                    wk<T>(c, 2))));
   }
