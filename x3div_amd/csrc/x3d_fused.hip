@@ -781,9 +781,12 @@ static int grad_pass(x3d_ctx* c, const S* a, const S* b, const S* cc, S* o1, S* 
   const PassArgs<S> A{a,    b,    cc,       o1,     o2,       o3,     ux,    uy,   uz,
                       s.cf_dpv, s.cc_s, s.cf_ipv, s.cc_i, s.geo, s.tl, corr, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
   if constexpr (!is_bfp<S>) {
-    // (x: outputs that a caller gave as one buffer are written in order)
-    if (split_pass<S>(c, s) && (DIR != 0 || (o1 != o2 && o1 != o3 && o2 != o3 && ux != o2 && ux != o3 && uy != o1 &&
-                                             uy != o3 && uz != o1 && uz != o2))) {
+    // (x: outputs that a caller gave as one buffer are written in order, and one
+    // buffer given for several velocities is corrected by all of them)
+    bool apart = true;
+    if constexpr (DIR == 0)
+      apart = corr ? outputs_apart<S>(c, {o1, o2, o3, ux, uy, uz}, {}) : outputs_apart<S>(c, {o1, o2, o3}, {});
+    if (apart && split_pass<S>(c, s)) {
       X3D_MSWITCH_T(S, s.M, hipLaunchKernelGGL((k_grad_split<S, MM, DIR>), dim3(s.grid.x, DIR == 2 ? 2 : 3), s.block,
                                                s.smem, c->stream, A));
       X3D_CHECK_HIP(hipGetLastError());
