@@ -42,3 +42,28 @@ def test_correction_in_order(torch_cuda, grid, form):
         for q in names:
             assert torch.equal(u[q], want[q]), (names, q)
     ctx.close()
+
+
+@pytest.mark.parametrize("form", ["f64", "f32"])
+@pytest.mark.parametrize("grid", GRIDS + [(32, 24, 320), (192, 40, 160)], **ids)
+def test_step_equals_its_passes(torch_cuda, grid, form):
+    """A step against the same step run as ten separate passes (the timed one),
+    with buffers apart and with a velocity's buffer given again: in both the
+    divergence is that of the velocities as all updates have left them."""
+    import torch
+    print(f"\n[step and its passes {grid} {form}]", flush=True)
+    ctx, u0, new = setup(grid, form)
+    step, timed = (ctx.step, ctx.step_timed) if form == "f64" else (ctx.step_f32, ctx.step_timed_f32)
+    # names of ux, uy, uz, dux, duy, duz
+    for names in ["uvwabc"] + [p + "abc" for p in PATTERNS] + ["uvwabu"]:
+        out = []
+        for run in (step, timed):
+            f = {q: u0[q].clone() if q in u0 else new() for q in names}
+            rest = [new() for _ in range(4)]
+            run(*(f[q] for q in names), *rest, gdt=1e-3)
+            out.append([f[q] for q in sorted(f)] + rest)
+        torch.cuda.synchronize()
+        for k, (a, b) in enumerate(zip(*out)):
+            assert torch.equal(a, b), (names, k)
+        assert bool(torch.isfinite(out[0][-1]).all()) and float(out[0][-1].abs().max()) > 0
+    ctx.close()

@@ -856,11 +856,13 @@ int fused_divergence(x3d_ctx* c, T* pp3, const T* ux, const T* uy, const T* uz)
 // -> 3.04 ms for the two, FP32 1.82 -> 1.51).  BFP32 keeps two passes: its x
 // passes are bound by the coder's instructions, and the fused one would code
 // u twice (2.53 -> 2.73 ms).  So does the per-pass timing (the same operations
-// on the same values), so that each pass has a time of its own.
+// on the same values), so that each pass has a time of its own, and a call that
+// gives a velocity's buffer again, as another velocity or a du: the fused pass
+// takes each velocity when its own update is done, before the later ones.
 template <typename T>
 int fused_momentum_divergence(x3d_ctx* c, double gdt, T* ux, T* uy, T* uz, T* dux, T* duy, T* duz, T* pp3)
 {
-  if (is_bfp<T> || c->timing) {
+  if (is_bfp<T> || c->timing || !outputs_apart<T>(c, {ux, uy, uz}, {dux, duy, duz})) {
     X3D_TRY(fused_momentum<T>(c, gdt, 1, ux, uy, uz, dux, duy, duz));
     return fused_divergence<T>(c, pp3, ux, uy, uz);
   }
