@@ -176,15 +176,10 @@ __device__ __forceinline__ void np_chunk_x(const double* in, const NpRows& r, co
   // kept by the chunk that holds it (every x wavefront holds both ends), and
   // zeros past the line's end
   if constexpr (RHS) {
-    const double x0 = np_rhs(win, H, 0, n, r);
-    if constexpr (M > 1) {
-      const double x1 = np_rhs(win, 1 + H, 1, n, r);
-      v[0] = c == 0 ? x0 : v[0];
-      v[1] = c == 0 ? x1 : v[1];
-    } else {
-      const double x1 = np_rhs(win, H, 1, n, r);
-      v[0] = c == 0 ? x0 : (c == 1 ? x1 : v[0]);
-    }
+    static_assert(M > 1, "the first chunk holds rows 0 and 1");
+    const double x0 = np_rhs(win, H, 0, n, r), x1 = np_rhs(win, 1 + H, 1, n, r);
+    v[0] = c == 0 ? x0 : v[0];
+    v[1] = c == 0 ? x1 : v[1];
 #pragma unroll
     for (int k = 0; k < M; ++k) {
       if (k == (n - 2) % M) {
@@ -656,13 +651,15 @@ NpRows np_rows(const x3d_ctx* c, int dir, int op)
 // two up to 64) of M <= 16 points with C M >= n and the least padding; x
 // counts chunks of more than 10 points a third longer, as their kernels hold
 // fewer wavefronts; y/z take up to 4 chunk groups per wavefront and C / 4
-// wavefronts per line set.
+// wavefronts per line set.  Chunks of half the points, twice as many, cover the
+// same points at no lower cost, so y/z chunks have 8 points or more and x ones,
+// where 11 or more may cost more than half of them, 6.
 int np_plan(int n, bool line_fast, LinePlan* P)
 {
   if (n < 8) return X3D_ERR_SIZE;
   int C = 0, M = 0, least = 1 << 30;
   for (int c = 1; c <= 64; c <<= 1)
-    for (int m = 1; m <= 16; ++m) {
+    for (int m = line_fast ? 8 : 6; m <= 16; ++m) {
       const int cost = c * m * (m > 10 && !line_fast ? 4 : 3);
       if (c * m >= n && cost < least) { C = c; M = m; least = cost; }
     }
@@ -705,20 +702,23 @@ int launch_line_np(x3d_ctx* c, int dir, int op, const double* in, double* out, b
   const double* tb = c->nptab + c->op[op].npoff;
   const OpDev<double> od{tb, tb + np, tb + 2 * np, nullptr, c->op[op].alfa};
   NpRows r = np_rows(c, dir, op);
-#define X3D_NP(MM)                                                                                            \
+#define X3D_NP(MM, LF)                                                                                        \
   case MM:                                                                                                    \
-    if (P.line_fast) {                                                                                        \
-      if (rhs) hipLaunchKernelGGL((k_der_np<MM, true, true>), grid, block, smem, c->stream, in, out, od, r, geo, tl); \
-      else hipLaunchKernelGGL((k_der_np<MM, true, false>), grid, block, smem, c->stream, in, out, od, r, geo, tl); \
-    } else {                                                                                                  \
-      if (rhs) hipLaunchKernelGGL((k_der_np<MM, false, true>), grid, block, smem, c->stream, in, out, od, r, geo, tl); \
-      else hipLaunchKernelGGL((k_der_np<MM, false, false>), grid, block, smem, c->stream, in, out, od, r, geo, tl); \
-    }                                                                                                         \
+    if (rhs) hipLaunchKernelGGL((k_der_np<MM, LF, true>), grid, block, smem, c->stream, in, out, od, r, geo, tl);  \
+    else hipLaunchKernelGGL((k_der_np<MM, LF, false>), grid, block, smem, c->stream, in, out, od, r, geo, tl);     \
     break;
-  switch (P.M) {
-    X3D_NP(1) X3D_NP(2) X3D_NP(3) X3D_NP(4) X3D_NP(5) X3D_NP(6) X3D_NP(7) X3D_NP(8)
-    X3D_NP(9) X3D_NP(10) X3D_NP(11) X3D_NP(12) X3D_NP(13) X3D_NP(14) X3D_NP(15) X3D_NP(16)
-    default: return X3D_ERR_UNSUPPORTED;
+  if (P.line_fast) {
+    switch (P.M) {
+      X3D_NP(8, true) X3D_NP(9, true) X3D_NP(10, true) X3D_NP(11, true) X3D_NP(12, true) X3D_NP(13, true)
+      X3D_NP(14, true) X3D_NP(15, true) X3D_NP(16, true)
+      default: return X3D_ERR_UNSUPPORTED;
+    }
+  } else {
+    switch (P.M) {
+      X3D_NP(6, false) X3D_NP(7, false) X3D_NP(8, false) X3D_NP(9, false) X3D_NP(10, false) X3D_NP(11, false)
+      X3D_NP(12, false) X3D_NP(13, false) X3D_NP(14, false) X3D_NP(15, false) X3D_NP(16, false)
+      default: return X3D_ERR_UNSUPPORTED;
+    }
   }
 #undef X3D_NP
   X3D_CHECK_HIP(hipGetLastError());
