@@ -132,18 +132,6 @@ int batch_step_body(x3d_batch* b, double gdt)
   return rc;
 }
 
-// Line lengths that this y/z tiling candidate fits, for the autotuner: the
-// chunk length M, chunk groups per wavefront G, line groups per work-group Wl.
-// LDS bytes of the largest pass (transeq, with its keep slots) for a y/z
-// tiling: solver aggregates (4 Wc + 2 lines per work-group when Wc > 1) plus
-// (2 M + 4) slots per thread.
-size_t plan_lds_bytes(const LinePlan& p, int prec)
-{
-  const size_t lpw = (size_t)p.Wl * p.LW, threads = 64u * p.Wc * p.Wl;
-  const size_t solver = p.Wc > 1 ? 4 * p.Wc * lpw + 2 * lpw : 0;
-  return (size_t)prec * (solver + threads * (size_t)(2 * p.M + 4));
-}
-
 // x-line tilings: chunks of M points, C = n / M chunks per line (a power of
 // two up to 64, so that a wavefront holds 64 / C whole lines), Wl wavefronts
 // per work-group, each with its LDS staging tile.
@@ -162,13 +150,14 @@ std::vector<LinePlan> candidates_x(int n, int prec, size_t lds_max)
     for (int wl : {1, 2, 4, 8}) {
       LinePlan p;
       p.n = n; p.M = m; p.C = c; p.G = c; p.Wc = 1; p.Wl = wl; p.LW = 64 / c; p.line_fast = false;
-      const size_t pitch = (m & 1) ? m : m + 1;
-      if ((size_t)prec * wl * 64 * pitch <= lds_max) out.push_back(p);
+      if (transeq_lds_bytes(p, (size_t)prec) <= lds_max) out.push_back(p);
     }
   }
   return out;
 }
 
+// y/z-line tilings: chunks of M points, G chunk groups per wavefront, Wl line
+// groups per work-group of at most 8 wavefronts.
 std::vector<LinePlan> candidates(int n, int prec, size_t lds_max)
 {
   static const int ms64[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
@@ -189,7 +178,7 @@ std::vector<LinePlan> candidates(int n, int prec, size_t lds_max)
         LinePlan p;
         p.n = n; p.M = m; p.C = c; p.G = g; p.Wc = wc; p.Wl = wl; p.LW = 64 / g; p.line_fast = true;
         p.bfp = p.LW % 16 == 0;
-        if (plan_lds_bytes(p, prec) <= lds_max) out.push_back(p);
+        if (transeq_lds_bytes(p, (size_t)prec) <= lds_max) out.push_back(p);
       }
     }
   }

@@ -477,6 +477,19 @@ void launch_dims(const x3d_ctx* c, int dir, Geom* geo, Tiling* tl, dim3* grid, d
   launch_dims_plan(c, dir, fused ? c->fplan[dir] : c->plan[dir], geo, tl, grid, block, smem, tbytes);
 }
 
+size_t line_lds_bytes(const LinePlan& P, size_t tbytes)
+{
+  // x-lines: one staging tile of 64 rows x (M or M+1, the odd one) per wavefront
+  if (!P.line_fast) return tbytes * (size_t)(P.Wc * P.Wl) * 64u * (size_t)((P.M & 1) ? P.M : P.M + 1);
+  return tbytes * (size_t)line_lds_words(P.Wc, P.Wl * P.LW);
+}
+
+size_t transeq_lds_bytes(const LinePlan& P, size_t tbytes)
+{
+  const size_t line = line_lds_bytes(P, tbytes);
+  return P.line_fast ? line + tbytes * (size_t)(64 * P.Wc * P.Wl) * (size_t)(P.M + 4) : 2 * line;
+}
+
 void launch_dims_plan(const x3d_ctx* c, int dir, const LinePlan& P, Geom* geo, Tiling* tl, dim3* grid,
                       dim3* block, size_t* smem, size_t tbytes)
 {
@@ -490,9 +503,7 @@ void launch_dims_plan(const x3d_ctx* c, int dir, const LinePlan& P, Geom* geo, T
   const int lpw = P.Wl * P.LW;
   *grid = dim3((geo->nlines + lpw - 1) / lpw);
   *block = dim3(64 * P.Wc * P.Wl);
-  *smem = tbytes * (size_t)line_lds_words(P.Wc, lpw);
-  // x-lines: one staging tile of 64 rows x (M or M+1, the odd one) per wavefront
-  if (!P.line_fast) *smem = tbytes * (size_t)(P.Wc * P.Wl) * 64u * (size_t)((P.M & 1) ? P.M : P.M + 1);
+  *smem = line_lds_bytes(P, tbytes);
 }
 
 template <typename S, int KIND, bool CIRC, typename T = typename Store<S>::T>

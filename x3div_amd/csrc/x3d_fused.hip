@@ -568,7 +568,7 @@ struct DirSet {
   Tiling tl;
   dim3 grid, block;
   size_t smem;
-  size_t smem_tq;  // transeq: plus the y/z keep slots
+  size_t smem_tq;  // transeq
   int M;
   Coef<T> cf_d, cf_dvp, cf_dpv, cf_ivp, cf_ipv;  // scaled by 1/gamma
   Circ<T> cc_d, cc_s, cc_i;
@@ -595,12 +595,7 @@ static DirSet<S> dirset(const x3d_ctx* c, int dir)
   if constexpr (is_bfp<S>)
     if (dir == 2) s.tl.xcd = c->xcd_remap;
   s.M = P.M;
-  // keep slots of transeq: the u_d window (M + 4)
-  s.smem_tq = s.smem;
-  if (P.line_fast)
-    s.smem_tq += sizeof(T) * (size_t)s.block.x * (size_t)(P.M + 4);
-  else
-    s.smem_tq = 2 * s.smem;  // x: the staging tile and the u_x tile
+  s.smem_tq = transeq_lds_bytes(P, sizeof(T));
   const Scheme& sc = c->sc[dir];
   // coefficients in FP64, rounded once to T
   auto scaled = [](Coef<double> k, double alfa) {

@@ -273,6 +273,11 @@ void launch_dims(const x3d_ctx* c, int dir, Geom* geo, Tiling* tl, dim3* grid, d
                  size_t tbytes, bool fused = false);
 void launch_dims_plan(const x3d_ctx* c, int dir, const LinePlan& P, Geom* geo, Tiling* tl, dim3* grid,
                       dim3* block, size_t* smem, size_t tbytes);
+// LDS bytes of a work-group: a line solve's (y/z: the solver's aggregates; x: a
+// staging tile per wavefront), and a transeq pass's, the largest of the step
+// (y/z: and the u_d window, M + 4 slots per thread; x: and the u_x tile).
+size_t line_lds_bytes(const LinePlan& P, size_t tbytes);
+size_t transeq_lds_bytes(const LinePlan& P, size_t tbytes);
 int line_plan_fused32(int n, bool line_fast, long long pts, LinePlan* out);
 // The fused plans of a context, FP64 and FP32, for launches of pts points (its
 // own, or those of the batch it belongs to).
