@@ -67,11 +67,15 @@ def profile_kernels(n: int, reps: int = 3):
     with torch.cuda.stream(ctx.stream):
         for _ in range(reps):
             t.copy_(f[0])
+    # the timed steps run transeq's and the divergence's x passes apart, which
+    # the FP64 and FP32 steps run as one
     for _ in range(reps):
         ctx.step(*f, gdt=0.0)
+        ctx.step_timed(*f, gdt=0.0)
     f32 = [t.float() for t in f[:3]] + [ctx.field32() for _ in range(7)]
     for _ in range(reps):
         ctx.step_f32(*f32, gdt=0.0)
+        ctx.step_timed_f32(*f32, gdt=0.0)
     del f32
     fb = [ctx.bfp_empty() for _ in range(10)]
     for i in range(3):
@@ -80,26 +84,33 @@ def profile_kernels(n: int, reps: int = 3):
         ctx.step_bfp(*fb, gdt=0.0)
     torch.cuda.synchronize()
     ctx.close()
-    print(f"profile-kernels: {n}^3, {reps} copies of {8 * n ** 3} B, {reps} FP64, {reps} FP32 and {reps} BFP32 steps",
-          flush=True)
+    print(f"profile-kernels: {n}^3, {reps} copies of {8 * n ** 3} B, {reps} FP64 and FP32 steps, as many timed ones, "
+          f"and {reps} BFP32 steps", flush=True)
 
 
 # the kernel template each line pass of the step launches
 KERNEL_OF_PASS = {
     "transeq_x": "k_transeq<double, M, 0>", "transeq_y": "k_transeq<double, M, 1>",
-    "transeq_z": "k_transeq<double, M, 2>", "divergence_x": "k_div<double, M, 0>",
+    "transeq_z": "k_transeq<double, M, 2>", "transeq_div_x": "k_transeq_div_x<double, M>",
+    "divergence_x": "k_div<double, M, 0>",
     "divergence_y": "k_div<double, M, 1>", "divergence_z": "k_div<double, M, 2>",
     "gradp_z": "k_grad<double, M, 2>", "gradp_y": "k_grad<double, M, 1>", "gradp_x": "k_grad<double, M, 0>",
 }
 
 
-def traffic_from_profile(pass_name: str, n: int):
-    """HBM bytes per launch of one pass's kernel from the committed PMC summary
-    (FETCH_SIZE + WRITE_SIZE, copy-calibrated), if one exists for this grid."""
+def kernel_of(pass_name: str, stype: str) -> str:
+    return KERNEL_OF_PASS[pass_name].replace("double", stype)
+
+
+def traffic_from_profile(pass_name: str, kernel: str, n: int):
+    """HBM bytes per launch of one pass's kernel (its name with M for the chunk
+    length) from the committed PMC summary (FETCH_SIZE + WRITE_SIZE,
+    copy-calibrated), if there is one for this grid and this kernel."""
     path = os.path.join(ROOT, "profiles", f"step_passes_{n}cubed_pmc.txt")
     if not os.path.exists(path):
         return None
-    m = re.search(rf"^hbm_bytes_per_launch\s+{pass_name}:\s*([0-9.eE+]+)", open(path).read(), re.M)
+    kern = re.escape(kernel).replace("M", r"\d+")
+    m = re.search(rf"^hbm_bytes_per_launch\s+{pass_name}\s+{kern}:\s*([0-9.eE+]+)", open(path).read(), re.M)
     return float(m.group(1)) if m else None
 
 
@@ -229,20 +240,33 @@ def measure_operators(ctx, src, dst, reps=10):
     return out
 
 
+def step_passes(passes, npts, gpu_ms_step, suffix):
+    """The passes that a step runs.  FP64 and FP32 steps apply the divergence's
+    x operators in the last transeq pass, so that u is not read again; the timed
+    step runs the two apart.  The one pass's time is what the other passes
+    leave of the step (at least 1 us: the events' own cost shows on the
+    smallest grids)."""
+    if suffix == "_bfp":
+        return passes
+    out = {k: p for k, p in passes.items() if k not in ("transeq_x", "divergence_x")}
+    ms = max(gpu_ms_step - sum(p["ms"] for p in out.values()), 1e-3)
+    bpp = passes["transeq_x"]["bytes_per_point"] + passes["divergence_x"]["bytes_per_point"] / 2
+    out["transeq_div_x"] = {"ms": round(ms, 4), "bytes_per_point": bpp,
+                            "GBps": round(bpp * npts / (ms / 1e3) / 1e9, 1), "from": "step - other passes"}
+    return out
+
+
 def roofline_of(passes, n, gpu_ms_step, suffix, npts=None, stype=None):
-    """The slowest line pass (the Poisson pass is several hipFFT kernels and is
+    """The step's slowest line pass (the Poisson pass is several kernels and is
     reported beside it) against the HBM peak, plus the whole step's fraction."""
     npts = npts or n ** 3
-    dom = max((k for k in passes if k != "poisson"), key=lambda k: passes[k]["ms"])
-    kms = passes[dom]["ms"]
-    alg_bytes = int(passes[dom]["bytes_per_point"] * npts)
+    run = step_passes(passes, npts, gpu_ms_step, suffix)
+    dom = max((k for k in run if k != "poisson"), key=lambda k: run[k]["ms"])
+    kms = run[dom]["ms"]
+    alg_bytes = int(run[dom]["bytes_per_point"] * npts)
     achieved = alg_bytes / (kms / 1e3) / 1e9
-    step_bytes = sum(p["bytes_per_point"] for p in passes.values()) * npts
-    if suffix != "_bfp":
-        # the step's last transeq pass also applies the divergence's x
-        # operators, so the step does not read u again (timed apart it does)
-        step_bytes -= passes["divergence_x"]["bytes_per_point"] / 2 * npts
-    kern = KERNEL_OF_PASS[dom].replace("double", stype or ("float" if suffix else "double"))
+    step_bytes = sum(p["bytes_per_point"] for p in run.values()) * npts
+    kern = kernel_of(dom, stype or ("float" if suffix else "double"))
     return {
         "bound": "hbm",
         "kernel": f"{dom} ({kern})",
@@ -250,12 +274,12 @@ def roofline_of(passes, n, gpu_ms_step, suffix, npts=None, stype=None):
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4),
-        "traffic": traffic_from_profile(dom + suffix, n),
+        "traffic": traffic_from_profile(dom + suffix, kern, n),
         "avg_launch_ms": round(kms, 4),
         "algorithmic_bytes_per_launch": alg_bytes,
         "step_algorithmic_bytes": int(step_bytes),
         "step_frac": round(step_bytes / (gpu_ms_step / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
-        "passes": passes,
+        "passes": {**passes, **run},
     }
 
 
