@@ -383,11 +383,13 @@ extern "C" int x3d_apply_circ_mfma(x3d_ctx* c, int op, float* out, const float* 
   // the input block too where both fit (and the wavefronts' maxima, 64 B)
   const bool stage = tsmem + bsmem <= 160 * 1024 - 256;
   const size_t smem = tsmem + (stage ? bsmem : 0);
-  // a wavefront per 64 output points (32 up to 256); as many persistent
-  // work-groups as the LDS and 16 wavefronts per compute unit allow
+  // a wavefront per 64 output points (32 up to 384); as many persistent
+  // work-groups as the LDS and 16 wavefronts per compute unit allow.  (384 by 6
+  // wavefronts of 64 points, which the four SIMDs do not share evenly, against
+  // 12 of 32: interpolation of 384 x 192 x 80 48 -> 18 us, derivative 23 -> 12)
   int& ncu = c->ncu;
   if (ncu <= 0) X3D_CHECK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
-  const int nw = n <= 256 ? n / 32 : n / 64;
+  const int nw = n <= 384 ? n / 32 : n / 64;
   const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(16 / nw, (160 * 1024) / (smem + 256)));
   const dim3 grid((unsigned)std::min(ntiles, ncu * per_cu));
 #define X3D_MFMA_RUN(NB, NW, XD, ST)                                                                             \
@@ -400,7 +402,7 @@ extern "C" int x3d_apply_circ_mfma(x3d_ctx* c, int op, float* out, const float* 
   } while (0)
 #define X3D_NB(NB)                                              \
   case NB: {                                                    \
-    constexpr int NW = NB <= 2 ? 4 * NB : 2 * NB;               \
+    constexpr int NW = NB <= 3 ? 4 * NB : 2 * NB;               \
     if (stage) {                                                \
       if (dir == 0) X3D_MFMA_RUN(NB, NW, true, true);           \
       else X3D_MFMA_RUN(NB, NW, false, true);                   \
