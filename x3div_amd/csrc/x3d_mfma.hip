@@ -56,6 +56,12 @@ struct CircBand {
   int lo, count;
 };
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 ld4(const float* base, unsigned boff, unsigned uniform = 0)
+{
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(field_rsrc(base), boff, uniform, 0));
+}
+
 // The fp16 halves of x, hi in the low 16 bits.
 __device__ __forceinline__ unsigned split_word(float x)
 {
@@ -94,7 +100,6 @@ __global__ __launch_bounds__(64 * NW) void k_circ_mfma(const float* __restrict__
   constexpr int n = 128 * NB, NT = 64 * NW, RB = n / (32 * NW), N16 = n / 16;
   static_assert(RB >= 1 && RB * 32 * NW == n, "whole row blocks per wavefront");
   constexpr int Q = 8 * n / NT;  // 16-byte loads of a tile per thread
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
   __shared__ float wmax[NW];
   __shared__ unsigned wbits[NW];
   // the operator's fragments (64 lanes x 32 B per offset) are read by every
@@ -119,8 +124,7 @@ __global__ __launch_bounds__(64 * NW) void k_circ_mfma(const float* __restrict__
       const unsigned off = first(tile) + (XDIR ? 16u * q : (q >> 3) * (rs * 4u) + 16u * (q & 7u));
 #pragma unroll
       for (int u = 0; u < Q; ++u)
-        x[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                             field_rsrc(in), off, u * (XDIR ? NT * 16u : (NT / 8) * rs * 4u), 0));
+        x[u] = ld4(in, off, u * (XDIR ? NT * 16u : (NT / 8) * rs * 4u));
     }
   };
   int tile = blockIdx.x;
@@ -152,8 +156,19 @@ __global__ __launch_bounds__(64 * NW) void k_circ_mfma(const float* __restrict__
         see(x[u].w);
       }
     } else {
-      // thread (lc, g) scans points g, g + NT / 32, ...
-      for (int k = threadIdx.x >> 5; k < n; k += NT / 32) see(ld(in, base + (unsigned)k * ps));
+      if constexpr (XDIR) {
+        // the 32 lines are one contiguous run
+        for (unsigned q = threadIdx.x; q < 8 * n; q += NT) {
+          const f32x4 y = ld4(in, t0 + 16u * q);
+          see(y.x);
+          see(y.y);
+          see(y.z);
+          see(y.w);
+        }
+      } else {
+        // thread (lc, g) scans points g, g + NT / 32, ...
+        for (int k = threadIdx.x >> 5; k < n; k += NT / 32) see(ld(in, base + (unsigned)k * ps));
+      }
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -220,8 +235,17 @@ __global__ __launch_bounds__(64 * NW) void k_circ_mfma(const float* __restrict__
         fl = __builtin_bit_cast(f16x8, l);
       } else {
         float y[8];
+        if constexpr (XDIR) {
+          const f32x4 a = ld4(in, base + (unsigned)(k0 + lk8) * 4u), b = ld4(in, base + (unsigned)(k0 + lk8) * 4u + 16u);
 #pragma unroll
-        for (int v = 0; v < 8; ++v) y[v] = ld(in, base + (unsigned)(k0 + lk8 + v) * ps) * scale;
+          for (int v = 0; v < 4; ++v) {
+            y[v] = a[v] * scale;
+            y[v + 4] = b[v] * scale;
+          }
+        } else {
+#pragma unroll
+          for (int v = 0; v < 8; ++v) y[v] = ld(in, base + (unsigned)(k0 + lk8 + v) * ps) * scale;
+        }
         split8(y, fh, fl);
       }
     };
