@@ -292,10 +292,13 @@ static int ew(x3d_ctx* c, int opk, double* o, const double* a, const double* b, 
 
 // The update loops of all three components in one launch: o_k = g a_k + o_k
 // (src/time_integrators.f90:42) or, SUB, o_k = o_k - a_k (src/navier.f90:84-86).
-// blockIdx.y is the component; each thread moves pairs of points by 16-byte
-// accesses (bases that are not 16-byte aligned take single points).  Bound by
-// HBM, 24 B per point and component: 320x96x160, one launch of 256-thread
-// blocks with 8-byte accesses per component 22 us each -> this 52 us for all (6.8 TB/s).
+// blockIdx.y is the component; each thread moves one point, or a pair by
+// 16-byte accesses.  Bound by the memory that holds the six fields: pairs while
+// the 256 MB cache holds most of them (320x96x160: 43 us, 8.2 TB/s; points 46;
+// one launch per component 52; 768x96x96, 340 MB: 67, 77, 87), points from
+// HBM on (256x256x128, 403 MB: pairs 98, points 97; 512^3: 1.57 ms, 6.2 TB/s;
+// pairs 1.67; one launch per component 1.73).  A grid of at most 16384 blocks that stride over
+// the fields takes 2.0 ms there, and 465 us instead of 391 at 512x512x128.
 template <bool SUB, bool PAIR>
 __global__ __launch_bounds__(256) void k_update3(double* o0, double* o1, double* o2, const double* a0, const double* a1,
                                                  const double* a2, double g, long long N)
@@ -303,18 +306,18 @@ __global__ __launch_bounds__(256) void k_update3(double* o0, double* o1, double*
   double* o = blockIdx.y == 0 ? o0 : (blockIdx.y == 1 ? o1 : o2);
   const double* a = blockIdx.y == 0 ? a0 : (blockIdx.y == 1 ? a1 : a2);
   auto f = [g](double x, double y) { return SUB ? y - x : g * x + y; };
-  const long long stride = (long long)gridDim.x * blockDim.x, first = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if constexpr (PAIR) {
-    for (long long q = first; q < N / 2; q += stride) {
+    if (q < N / 2) {
       const double2 x = reinterpret_cast<const double2*>(a)[q];
       double2 y = reinterpret_cast<double2*>(o)[q];
       y.x = f(x.x, y.x);
       y.y = f(x.y, y.y);
       reinterpret_cast<double2*>(o)[q] = y;
     }
-    if (first == 0 && N % 2) o[N - 1] = f(a[N - 1], o[N - 1]);
+    if (q == 0 && N % 2) o[N - 1] = f(a[N - 1], o[N - 1]);
   } else {
-    for (long long q = first; q < N; q += stride) o[q] = f(a[q], o[q]);
+    if (q < N) o[q] = f(a[q], o[q]);
   }
 }
 
@@ -322,7 +325,7 @@ template <bool SUB>
 static int update3(x3d_ctx* c, double* const (&o)[3], const double* const (&a)[3], double g)
 {
   const long long N = (long long)c->nx * c->ny * c->nz;
-  bool pair = true, apart = true;
+  bool pair = 6 * 8 * N < 384LL << 20, apart = true;
   for (int k = 0; k < 3; ++k) {
     pair = pair && !((reinterpret_cast<uintptr_t>(o[k]) | reinterpret_cast<uintptr_t>(a[k])) & 15);
     for (int l = 0; l < 3; ++l)
@@ -331,7 +334,7 @@ static int update3(x3d_ctx* c, double* const (&o)[3], const double* const (&a)[3
   const long long per = pair ? 512 : 256;
   // a component that updates another's operand (one buffer given for two of
   // them): the components in order, one launch each
-  const dim3 grid((unsigned)std::min<long long>((N + per - 1) / per, 16384), apart ? 3 : 1);
+  const dim3 grid((unsigned)((N + per - 1) / per), apart ? 3 : 1);
   for (int k = 0; k < (apart ? 1 : 3); ++k) {
     const int k1 = apart ? 1 : k, k2 = apart ? 2 : k;
     if (pair)
