@@ -50,7 +50,10 @@ struct Coef { T a, b, c, d; };
 // The fused multiply-adds are written out: which of two products the compiler
 // fuses into their sum depends on the code around it, and kernels that compute
 // the same values (a fused pass and the passes it stands for) would differ in
-// their last bits.
+// their last bits.  The third and fourth terms of the interpolations, one
+// product and one sum each, leave no choice, and stay plain sums: as nested
+// fused multiply-adds they cost the 16-point y and z kernels a spilled register
+// (512^3: y 393 -> 407 us, z 498 -> 521).
 template <int KIND, typename T>
 __device__ __forceinline__ T rhs_at(const T* win, int q, const Coef<T>& k)
 {
@@ -61,11 +64,11 @@ __device__ __forceinline__ T rhs_at(const T* win, int q, const Coef<T>& k)
   else if constexpr (KIND == K_DPV)
     return fma(k.a, win[q] - win[q - 1], k.b * (win[q + 1] - win[q - 2]));
   else if constexpr (KIND == K_IVP)
-    return fma(k.d, win[q + 4] + win[q - 3], fma(k.c, win[q + 3] + win[q - 2],
-               fma(k.a, win[q + 1] + win[q], k.b * (win[q + 2] + win[q - 1]))));
+    return fma(k.a, win[q + 1] + win[q], k.b * (win[q + 2] + win[q - 1])) + k.c * (win[q + 3] + win[q - 2]) +
+           k.d * (win[q + 4] + win[q - 3]);
   else if constexpr (KIND == K_IPV)
-    return fma(k.d, win[q + 3] + win[q - 4], fma(k.c, win[q + 2] + win[q - 3],
-               fma(k.a, win[q] + win[q - 1], k.b * (win[q + 1] + win[q - 2]))));
+    return fma(k.a, win[q] + win[q - 1], k.b * (win[q + 1] + win[q - 2])) + k.c * (win[q + 2] + win[q - 3]) +
+           k.d * (win[q + 3] + win[q - 4]);
   else if constexpr (KIND == K_DD)
     return fma(k.a, fma((T)-2, win[q], win[q + 1] + win[q - 1]), k.b * fma((T)-2, win[q], win[q + 2] + win[q - 2]));
   else
