@@ -670,10 +670,16 @@ static bool storage_ok(const x3d_ctx* c, int dir)
 // need fewer registers, up to 7 (64 x 128 x 192 167 -> 162; at 8, 160^3 327 ->
 // 333).  Same arithmetic per output, so the results are bit for bit the same.
 // BFP32 fields keep one launch shape.
+// Transeq's three components have to find room at once: its FP64 passes of
+// 16-point chunks, at 2 wavefronts per SIMD, stop at 3 per compute unit.  us for
+// the pass, whole -> split: y of 64 x 128 x 96 (3 wavefronts) 20.2 -> 18.4, of 64
+// x 160 x 96 (3.75) 24.4 -> 26.0, of 64 x 128 x 128 (4) 22.0 -> 22.9, of 24 x 320
+// x 160 (4.7) 27.8 -> 37.5; 12-point chunks, z of 64 x 160 x 96 (5) 19.9 -> 18.4.
 template <typename S>
-static bool split_pass(const x3d_ctx* c, const DirSet<S>& s)
+static bool split_pass(const x3d_ctx* c, const DirSet<S>& s, bool transeq = false)
 {
-  const int waves_per_cu = sizeof(typename Store<S>::T) == 8 ? 5 : 7;
+  constexpr bool f64 = sizeof(typename Store<S>::T) == 8;
+  const int waves_per_cu = !f64 ? 7 : transeq && s.M >= 16 ? 3 : 5;
   return !is_bfp<S> && (long long)s.grid.x * (s.block.x / 64) <= waves_per_cu * (long long)c->ncu;
 }
 
@@ -705,7 +711,7 @@ static int transeq_pass(x3d_ctx* c, S* ux, S* uy, S* uz, S* dux, S* duy, S* duz,
                          ty,   tz,   s.cf_d, s.cc_d, s.geo, s.tl, (T)gdt,
                          euler, DIR == 1 ? stretch_vec<T>(c, 0) : nullptr};
   if constexpr (DIR != 0 && !is_bfp<S>) {
-    if (apart && split_pass<S>(c, s)) {
+    if (apart && split_pass<S>(c, s, true)) {
       X3D_MSWITCH_T(S, s.M, {
         allow_lds((const void*)k_transeq_split<S, MM, DIR>, s.smem_tq);
         hipLaunchKernelGGL((k_transeq_split<S, MM, DIR>), dim3(s.grid.x, 3), s.block, s.smem_tq, c->stream, A);
