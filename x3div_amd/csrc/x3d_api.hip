@@ -237,9 +237,10 @@ int fused_plans(x3d_ctx* c, long long pts)
   for (int d = 0; d < 3; ++d) ok32 = !line_plan_fused32(ns[d], d != 0, pts, &c->fplan32[d]) && ok32;
   if (!ok32) c->fplan32[0].M = c->fplan32[1].M = c->fplan32[2].M = 0;
   for (int d = 0; d < 3; ++d) {
-    const int rc = line_plan_fused(ns[d], d != 0, pts, &c->fplan[d], variant);
+    int rc = line_plan_fused(ns[d], d != 0, pts, &c->fplan[d], variant, false);
+    if (!rc) rc = line_plan_fused(ns[d], d != 0, pts, &c->bplan[d], variant, true);
     if (rc && !c->ncl1[d]) return rc;
-    if (rc) c->fplan[d] = LinePlan{};
+    if (rc) c->fplan[d] = c->bplan[d] = LinePlan{};
   }
   return X3D_OK;
 }

@@ -326,9 +326,9 @@ static bool x_tiling(int n, int cap, const int (&ms)[K], LinePlan* p)
 // the cap or more, in pairs; for FP32 long chunks in any number (one group);
 // then the longest with whole groups.  (FP64 160: 10 chunks of 16 points as
 // pairs 332 us for the six y and z passes, 20 of 8 points 361; 96: 8 of 12
-// points 99 us, 32 of 3 points 155.)
+// points 99 us, 32 of 3 points 155.)  pair: the shortest chunks that go in pairs.
 template <int K>
-static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p)
+static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p, int pair = 0)
 {
   for (int pass = 0; pass < 5; ++pass)
     for (int q = K - 1; q >= 0; --q) {
@@ -342,7 +342,7 @@ static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p)
         g = 1;
       }
       if (pass == 3) {
-        if (c % 2 || 2 * m < cap) continue;
+        if (c % 2 || 2 * m < cap || (c % g0 && m < pair)) continue;
         g = c % g0 ? 2 : g0;
       }
       if (pass == 4 && c % g0) continue;
@@ -357,9 +357,29 @@ static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p)
 // points instead of 16 below 512 wavefronts (two per compute unit); FP32 32
 // points from 1600 wavefronts on, 8 below 100.
 // (a line that 8-point chunks do not tile, 320 points, takes the longer ones)
-static bool yz_tiling64(int n, long long pts, LinePlan* p)
+// BFP32 passes pair 16-point chunks alone: 80 points, 16 chunks of 5 / 10 of 8
+// as pairs, us for the three passes of a direction: y and z of 160 x 80 x 80 119
+// / 134, z of 384 x 192 x 80 170 / 218, y of 32 x 80 x 24 44 / 49.
+static bool yz_tiling64(int n, long long pts, LinePlan* p, bool bfp = false)
 {
-  return (pts / (64 * 16) < 512 && yz_tiling(n, 8, 4, kMs, p)) || yz_tiling(n, 16, 4, kMs, p);
+  const int pair = bfp ? 16 : 0;
+  return (pts / (64 * 16) < 512 && yz_tiling(n, 8, 4, kMs, p, pair)) || yz_tiling(n, 16, 4, kMs, p, pair);
+}
+
+// BFP32 x-lines: half the chunk while it leaves fewer than 1536 wavefronts (six
+// per compute unit), down to 2 points.  Their coder's instructions grow with
+// the chunk, and no pass of theirs is split.  us for the three x passes, 8 / 4 /
+// 2 points: 64 x 40 x 40 45.8 / 39.5 / 37.2, 64^3 49.3 / 43.4 / 43.0, 128 x 64 x
+// 64 (1024 wavefronts of 8) 55.2 / 51.4 / 57.5, 256 x 64 x 64 (2048) 63.1 / 65.0,
+// 128 x 96 x 96 (2304) 68.7 / 68.7, 128^3 81 / 96.
+static void bfp_x_chunk(long long pts, LinePlan* p)
+{
+  while (p->M % 2 == 0 && p->M > 2 && p->C <= 32 && pts / (64 * p->M) < 1536) {
+    p->M /= 2;
+    p->C *= 2;
+  }
+  p->G = p->C;
+  p->LW = 64 / p->C;
 }
 static int yz_cap32(long long pts) { return pts / (64 * 32) >= 1600 ? 32 : (pts / (64 * 16) >= 100 ? 16 : 8); }
 
@@ -400,9 +420,13 @@ int line_plan(int n, bool line_fast, long long pts, LinePlan* P)
 // work-group at 8 wavefronts (up to 256 VGPRs each): yz_tiling, else the
 // largest C <= 32 chunks per line with 4 chunk groups x 16 lines per
 // wavefront, else 64 chunks with 8 groups x 8 lines.
-int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* P, int variant)
+int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* P, int variant, bool bfp)
 {
-  if (!line_fast) return line_plan(n, false, pts, P);
+  if (!line_fast) {
+    const int rc = line_plan(n, false, pts, P);
+    if (!rc && bfp) bfp_x_chunk(pts, P);
+    return rc;
+  }
   if (n < 8) return X3D_ERR_SIZE;
   auto okM = [](int m) { return has_chunk(kMs, m); };
   LinePlan p;
@@ -432,14 +456,14 @@ int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* P, int varia
     if (n % c || !okM(n / c)) continue;
     p.C = c; p.M = n / c; p.G = c < 4 ? c : 4; p.Wc = c / p.G;
     p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc; p.LW = 64 / p.G;
-    (void)yz_tiling64(n, pts, &p);
+    (void)yz_tiling64(n, pts, &p, bfp);
     p.bfp = p.LW % 16 == 0;
     *P = p;
     return X3D_OK;
   }
   if (n % 64 == 0 && okM(n / 64)) {
     p.C = 64; p.M = n / 64; p.G = 8; p.Wc = 8; p.Wl = 1; p.LW = 8;
-    (void)yz_tiling64(n, pts, &p);
+    (void)yz_tiling64(n, pts, &p, bfp);
     *P = p;
     return X3D_OK;
   }

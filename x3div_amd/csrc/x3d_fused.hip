@@ -579,7 +579,7 @@ struct DirSet {
 template <typename S>
 static const LinePlan& fused_plan(const x3d_ctx* c, int dir)
 {
-  return std::is_same<S, float>::value ? c->fplan32[dir] : c->fplan[dir];
+  return is_bfp<S> ? c->bplan[dir] : std::is_same<S, float>::value ? c->fplan32[dir] : c->fplan[dir];
 }
 
 template <typename S>

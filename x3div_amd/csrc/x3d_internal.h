@@ -89,6 +89,7 @@ struct x3d_ctx {
   x3d::LinePlan plan[3];   // single-operator kernels
   x3d::LinePlan fplan[3];  // fused step passes (at most 512 threads per work-group)
   x3d::LinePlan fplan32[3];  // fused step passes of the FP32 precision form
+  x3d::LinePlan bplan[3];  // fused step passes of the BFP32 form
   // Poisson
   hipfftHandle fft_r2c = 0, fft_c2r = 0;
   bool fft_ready = false;
@@ -214,7 +215,7 @@ int batch_fork(x3d_batch* b);
 int batch_join(x3d_batch* b, int rc);
 // Line tilings for lines of n points; pts: the points one launch covers.
 int line_plan(int n, bool line_fast, long long pts, LinePlan* out);
-int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* out, int variant);
+int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* out, int variant, bool bfp);
 
 // Launch one compact operator (or Thomas alone) along direction dir.
 int launch_line_f32(x3d_ctx* c, int dir, int kind, int op, const float* in, float* out);
@@ -279,7 +280,7 @@ void launch_dims_plan(const x3d_ctx* c, int dir, const LinePlan& P, Geom* geo, T
 size_t line_lds_bytes(const LinePlan& P, size_t tbytes);
 size_t transeq_lds_bytes(const LinePlan& P, size_t tbytes);
 int line_plan_fused32(int n, bool line_fast, long long pts, LinePlan* out);
-// The fused plans of a context, FP64 and FP32, for launches of pts points (its
+// The fused plans of a context, FP64, FP32 and BFP32, for launches of pts points (its
 // own, or those of the batch it belongs to).
 int fused_plans(x3d_ctx* c, long long pts);
 
