@@ -357,13 +357,16 @@ static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p, i
 // points instead of 16 below 512 wavefronts (two per compute unit); FP32 32
 // points from 1600 wavefronts on, 8 below 100.
 // (a line that 8-point chunks do not tile, 320 points, takes the longer ones)
-// BFP32 passes pair 16-point chunks alone: 80 points, 16 chunks of 5 / 10 of 8
-// as pairs, us for the three passes of a direction: y and z of 160 x 80 x 80 119
-// / 134, z of 384 x 192 x 80 170 / 218, y of 32 x 80 x 24 44 / 49.
-static bool yz_tiling64(int n, long long pts, LinePlan* p, bool bfp = false)
+// Fused passes pair 16-point chunks alone, but for small FP64 grids, whose
+// passes are split.  80 points, 16 chunks of 5 / 10 of 8 as pairs, us for the
+// three passes of a direction: FP64 y and z of 160 x 80 x 80 115 / 118 (transeq
+// 48 / 55), BFP32 119 / 134, z of 384 x 192 x 80 170 / 218, y of 32 x 80 x 24 44
+// / 49.
+enum Pairs { PAIRS_ANY, PAIRS_F64, PAIRS_BFP };
+static bool yz_tiling64(int n, long long pts, LinePlan* p, Pairs pairs = PAIRS_ANY)
 {
-  const int pair = bfp ? 16 : 0;
-  return (pts / (64 * 16) < 512 && yz_tiling(n, 8, 4, kMs, p, pair)) || yz_tiling(n, 16, 4, kMs, p, pair);
+  return (pts / (64 * 16) < 512 && yz_tiling(n, 8, 4, kMs, p, pairs == PAIRS_BFP ? 16 : 0)) ||
+         yz_tiling(n, 16, 4, kMs, p, pairs == PAIRS_ANY ? 0 : 16);
 }
 
 // BFP32 x-lines: half the chunk while it leaves fewer than 1536 wavefronts (six
@@ -456,14 +459,14 @@ int line_plan_fused(int n, bool line_fast, long long pts, LinePlan* P, int varia
     if (n % c || !okM(n / c)) continue;
     p.C = c; p.M = n / c; p.G = c < 4 ? c : 4; p.Wc = c / p.G;
     p.Wl = p.Wc >= 4 ? 1 : 4 / p.Wc; p.LW = 64 / p.G;
-    (void)yz_tiling64(n, pts, &p, bfp);
+    (void)yz_tiling64(n, pts, &p, bfp ? PAIRS_BFP : PAIRS_F64);
     p.bfp = p.LW % 16 == 0;
     *P = p;
     return X3D_OK;
   }
   if (n % 64 == 0 && okM(n / 64)) {
     p.C = 64; p.M = n / 64; p.G = 8; p.Wc = 8; p.Wl = 1; p.LW = 8;
-    (void)yz_tiling64(n, pts, &p, bfp);
+    (void)yz_tiling64(n, pts, &p, bfp ? PAIRS_BFP : PAIRS_F64);
     *P = p;
     return X3D_OK;
   }
