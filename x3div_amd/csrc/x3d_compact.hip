@@ -357,6 +357,13 @@ static bool yz_tiling(int n, int cap, int g0, const int (&ms)[K], LinePlan* p, i
 // points instead of 16 below 512 wavefronts (two per compute unit); FP32 32
 // points from 1600 wavefronts on, 8 below 100.
 // (a line that 8-point chunks do not tile, 320 points, takes the longer ones)
+// Small grids run their passes split by output, which leaves little between
+// the caps around these lines.  us per step, shorter / longer chunks, by
+// wavefronts of the longer: FP64 32 66.2 / 66.1, 108 82.8 / 79.9, 256 97.9 /
+// 97.3, 500 137.6 / 137.5, 576 140.1 / 132.3, 864 175 / 161, 2048 285 / 277;
+// FP32 16 against 32 points 1024 187 / 184, 1440 236 / 232, 1600 273 / 270,
+// 2000 363 / 328, 4096 536 / 514; 8 against 16 points 32 62.1 / 62.1, 96 68.7
+// / 68.0, 108 70.6 / 69.0, 256 80.6 / 80.3, 500 104.8 / 107.4.
 // Fused passes pair 16-point chunks alone, but for small FP64 grids, whose
 // passes are split.  80 points, 16 chunks of 5 / 10 of 8 as pairs, us for the
 // three passes of a direction: FP64 y and z of 160 x 80 x 80 115 / 118 (transeq
@@ -692,6 +699,9 @@ NpRows np_rows(const x3d_ctx* c, int dir, int op)
 // wavefronts per line set.  Chunks of half the points, twice as many, cover the
 // same points at no lower cost, so y/z chunks have 8 points or more and x ones,
 // where 11 or more may cost more than half of them, 6.
+// (derx of n x 128 x 256, us, without / with the third: n = 43 8.5 / 8.0, 171
+// 23.5 / 24.2, 240 36.7 / 29.9, 350 40.5 / 43.7, 400 45.3 / 47.1, 440 58.0 /
+// 49.2, 470 69.7 / 56.0, 500 64.2 / 56.9.)
 int np_plan(int n, bool line_fast, LinePlan* P)
 {
   if (n < 8) return X3D_ERR_SIZE;

@@ -472,7 +472,9 @@ __device__ __forceinline__ int grid_of(const int* __restrict__ block0, int ngrid
 template <typename S, int M, int DIR>
 __global__ __launch_bounds__(512) void k_transeq(TranseqArgs<S> A) { transeq_body<S, M, DIR>(A, A.tl.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x); }
 // (held to the registers of the pass without the divergence: FP64 chunks of 8
-// points would take 131 and leave 3 wavefronts per SIMD, of 12 points 172 and 2)
+// points would take 131 and leave 3 wavefronts per SIMD, of 12 points 172 and
+// 2.  The spills move 7% more bytes at 512^3.  Steps without / with the cap:
+// 128^3 284 / 278 us, 256^3 1.876 / 1.886 ms, 512^3 15.95 ms either way)
 template <typename S, int M>
 constexpr int divx_waves() { return sizeof(S) == 8 ? (M <= 8 ? 4 : M <= 12 ? 3 : 1) : 1; }
 template <typename S, int M>
