@@ -220,7 +220,10 @@ int x3d_poisson(x3d_ctx *ctx, double *rhs);
 int x3d_poisson_tables(const x3d_ctx *ctx, double *ax, double *bx, double *ay, double *by,
                        double *az, double *bz, double *kxyz_re);
 
-/* ---- timestep pieces (callers of the operators) ----------------------- */
+/* ---- timestep pieces (callers of the operators) -----------------------
+ * A buffer given for several outputs of one call is written in the order x, y,
+ * z (the last one stays), one given for several velocities takes each of their
+ * updates and corrections in that order. */
 /* calculate_transeq_rhs / momentum_rhs_eq (src/transeq.f90:18-355) */
 int x3d_momentum_rhs(x3d_ctx *ctx, double *dux, double *duy, double *duz,
                      const double *ux, const double *uy, const double *uz);

@@ -177,7 +177,6 @@ std::vector<LinePlan> candidates(int n, int prec, size_t lds_max)
         if (wc * wl > 8) continue;
         LinePlan p;
         p.n = n; p.M = m; p.C = c; p.G = g; p.Wc = wc; p.Wl = wl; p.LW = 64 / g; p.line_fast = true;
-        p.bfp = p.LW % 16 == 0;
         if (transeq_lds_bytes(p, (size_t)prec) <= lds_max) out.push_back(p);
       }
     }

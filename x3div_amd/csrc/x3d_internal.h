@@ -65,7 +65,7 @@ struct LinePlan {
   int Wl = 0;     // independent line groups per work-group
   int LW = 0;     // lines per wavefront (64 / G)
   bool line_fast = false;  // lanes: consecutive lines (y/z) or consecutive chunks (x)
-  bool bfp = false;  // fused y/z: the BFP32 step takes the line (one of at most 32 chunks, whole 16-line rows)
+  bool bfp = false;  // BFP32 step, y/z: it takes the line (a power of two of at most 32 chunks divides it; whole 16-line rows)
 };
 
 }  // namespace x3d
