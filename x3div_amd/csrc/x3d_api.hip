@@ -295,11 +295,12 @@ static int ew(x3d_ctx* c, int opk, double* o, const double* a, const double* b, 
 // (src/time_integrators.f90:42) or, SUB, o_k = o_k - a_k (src/navier.f90:84-86).
 // blockIdx.y is the component; each thread moves one point, or a pair by
 // 16-byte accesses.  Bound by the memory that holds the six fields: pairs while
-// the 256 MB cache holds most of them (320x96x160: 43 us, 8.2 TB/s; points 46;
-// one launch per component 52; 768x96x96, 340 MB: 67, 77, 87), points from
-// HBM on (256x256x128, 403 MB: pairs 98, points 97; 512^3: 1.57 ms, 6.2 TB/s;
-// pairs 1.67; one launch per component 1.73).  A grid of at most 16384 blocks that stride over
-// the fields takes 2.0 ms there, and 465 us instead of 391 at 512x512x128.
+// the 256 MB cache holds most of them, points from HBM on (the kernel alone,
+// pairs / points: 320x96x160 43 / 46 us, 768x96x96 67 / 77, 256x256x128, 403 MB,
+// 98 / 97, 512^3 1.67 / 1.57 ms).  The call, one launch per component -> this:
+// 320x96x160 57 -> 48 us, 512x512x128 403 -> 391, 512^3 1.74 -> 1.61 ms (6.0
+// TB/s).  A grid of at most 16384 blocks that stride over the fields: 464 us
+// and 2.04 ms at the last two.
 template <bool SUB, bool PAIR>
 __global__ __launch_bounds__(256) void k_update3(double* o0, double* o1, double* o2, const double* a0, const double* a1,
                                                  const double* a2, double g, long long N)
